@@ -97,6 +97,41 @@ struct ZTendArgs {
     const double *extra[3];   // optional mixed-spectral tendency added to the source (closure)
 };
 
+// One z pass of an RK4 step on the semi-spectral state (k_zstage*).
+//
+// Everything between the horizontal transforms is linear per column, and the
+// decompositions of vorticity_tendency (five DSTs per column and stage) only undo the
+// combines that the next vor2vel starts with (five more).  The steps therefore keep the
+// state combined -- in svor, also between steps: turning it into the mixed form and back
+// adds the transforms' rounding to the state itself, which over 20 steps at 256^3 made
+// the error against 64-bit arithmetic eight times larger -- and a stage is left with the
+// transforms of the Poisson solve for w.
+// Kind of pass: ZS_START vor2vel of svor; ZS_STAGE1 / ZS_STAGE23 tendency, substep and
+// the next stage's vor2vel; ZS_STAGE4 tendency, last substep, mean restore and time
+// update; ZS_STEP the first substep from a stored mixed tendency (source, then step).
+enum { ZS_START = 0, ZS_STAGE1 = 1, ZS_STAGE23 = 2, ZS_STAGE4 = 4, ZS_STEP = 5 };
+struct ZStageArgs {
+    Grid g;
+    ZTabs tb;
+    int TQ, QPB, nquads;
+    FftPlan pz;
+    const double2 *twz;
+    double zscale, rkz_sc;
+    int stage;                // ZS_STAGE23: 2 or 3
+    // horizontal wavenumber indices up to kxb, kyb pass the tendency filter; beyond
+    // them it is exactly zero (2/3 rule), r, q and p are not read and the state only
+    // decays.  nx/2, ny/2: every column is in the band.
+    int kxb, kyb;
+    const double *in[3];      // ZS_STEP: svorts (mixed); ZS_STAGE*: r, q, p (semi-spectral)
+    double *svor[3];          // the state at the step's start; ZS_STAGE4 writes the new one
+    double *qdf[3];           // the accumulated result
+    double *out[6];           // u, v, w, xi, eta, zeta; ZS_START: out[3..5] = svor (projected)
+    double *mid[3];           // ZS_START: z-midpoint vorticity, or nullptr
+    const double *extra[3];   // optional semi-spectral tendency added to the source (closure)
+    double *scal;
+    Batch bt;
+};
+
 struct ZOpArgs {
     Grid g;
     ZTabs tb;
@@ -125,6 +160,7 @@ hipError_t launch_zinv(const ZLaunch &zl, const ZInvArgs &args, hipStream_t stre
 hipError_t launch_ztend(const ZLaunch &zl, const ZTendArgs &args, hipStream_t stream);
 hipError_t launch_zrk(const ZLaunch &zl, const ZTendArgs &args, hipStream_t stream);
 hipError_t launch_zop(const ZLaunch &zl, const ZOpArgs &args, hipStream_t stream);
+hipError_t launch_zstage(const ZLaunch &zl, int kind, const ZStageArgs &args, hipStream_t stream);
 
 // wave-per-column z kernels (zwave.hip), nz in {128, 256, 512}
 bool zwave_supported(int nz);
@@ -135,10 +171,7 @@ hipError_t configure_zwave();
 hipError_t launch_zinv_w(int nz, int variant, int nquads, const ZInvArgs &args, hipStream_t stream);
 hipError_t launch_ztend_w(int nz, int variant, int nquads, const ZTendArgs &args, hipStream_t stream);
 hipError_t launch_zop_w(int nz, int nquads, const ZOpArgs &args, hipStream_t stream);
-// RK4 stage 1..3 of the tendency pass fused with the next stage's vor2vel pass (the
-// stage result stays in registers; t.rk.q is not written)
-hipError_t launch_ztend_zinv_w(int nz, int variant, int nquads, const ZTendArgs &t, const ZInvArgs &z,
-                               hipStream_t stream);
+hipError_t launch_zstage_w(int nz, int nquads, int kind, const ZStageArgs &args, hipStream_t stream);
 hipError_t launch_mean(const MeanArgs &args, int nz, hipStream_t stream);
 
 // Pointwise kernels of the output-step derived fields (fields_derived.f90:67-182),

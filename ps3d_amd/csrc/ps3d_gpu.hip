@@ -74,7 +74,11 @@ struct ps3d_handle {
     FftPlan px{}, py{}, pz{};
     ZLaunch zl{};
     int TQ = 0, QPB = 0, nquads = 0;
-    bool zfuse = true;             // RK4 tendency pass fused with the next vor2vel pass
+    // RK4 steps on the semi-spectral state (launch_zstage); PS3D_ZFUSE=0 keeps the
+    // passes of the operator entry points, vor2vel and tendency on svor, for comparison
+    bool zfuse = true;
+    bool svor_semi = false;        // svor holds combined columns (between such steps)
+    int kxb = 0, kyb = 0;          // largest wavenumber indices the tendency filter passes
     LineCfg lx{}, ly{};
     // tiles of the register-holding line modes (x products pass lxm, x adapt pass lxr,
     // adapt-stage y pass lyr) and their block sizes: 1024 threads on the standard
@@ -329,6 +333,13 @@ static int init_handle(ps3d_handle *h, const ps3d_params *p, bool alloc_fields, 
         for (int k = 0; k < ny; ++k) fy[k] = (h->h_rky[k] <= f23 * my) ? 1.0 : 0.0;
         for (int k = 0; k <= nz; ++k) fz[k] = (rkz[k] <= f23 * mz) ? 1.0 : 0.0;
     }
+    // the 2/3 rule is exactly zero beyond a wavenumber index, the other filter nowhere
+    h->kxb = nx / 2;
+    h->kyb = ny / 2;
+    if (p->filtering == PS3D_FILTER_23RULE) {
+        while (h->kxb > 0 && fx[h->kxb] == 0.0) --h->kxb;
+        while (h->kyb > 0 && fy[h->kyb] == 0.0) --h->kyb;
+    }
     int st;
     if ((st = upload(&h->rkx, h->h_rkx)) || (st = upload(&h->rky, h->h_rky)) || (st = upload(&h->filx, fx)) ||
         (st = upload(&h->fily, fy)) || (st = upload(&h->filz, fz)))
@@ -580,6 +591,35 @@ static ZTendArgs ztend_args(ps3d_handle *h, int mode, int stage, double *const *
     return a;
 }
 
+// z pass of an RK4 step on the semi-spectral state: svor holds the combined state of the
+// step's start, qdf the accumulated result.  in: r, q, p or svorts; nullptr: ZS_START.
+static ZStageArgs zstage_args(ps3d_handle *h, int stage, double *const *in) {
+    ZStageArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.g = h->g;
+    a.tb = ztabs(h);
+    a.TQ = h->TQ;
+    a.QPB = h->QPB;
+    a.nquads = h->nquads;
+    a.pz = h->pz;
+    a.twz = h->twz;
+    a.zscale = 1.0 / std::sqrt(2.0 * h->g.nz);
+    a.rkz_sc = 3.141592653589793238462643383279502884 / h->p.extent[2];
+    a.stage = stage;
+    a.kxb = h->kxb;
+    a.kyb = h->kyb;
+    for (int c = 0; c < 3; ++c) {
+        a.in[c] = in ? in[c] : nullptr;
+        a.qdf[c] = h->qdf[c];
+        a.svor[c] = h->svor[c];
+        a.out[c] = h->svel[c];
+        a.out[3 + c] = in ? h->vor[c] : h->svor[c];
+    }
+    a.scal = h->scal;
+    a.bt = batch(h);
+    return a;
+}
+
 static ZOpArgs zop_args(ps3d_handle *h, int op, const double *in, double *out) {
     ZOpArgs a;
     std::memset(&a, 0, sizeof a);
@@ -598,15 +638,15 @@ static ZOpArgs zop_args(ps3d_handle *h, int op, const double *in, double *out) {
     return a;
 }
 
-static int run_mean(ps3d_handle *h, int mode, int advance_time) {
+static int run_mean(ps3d_handle *h, int mode, int advance_time, double *const *svor = nullptr) {
     MeanArgs a;
     std::memset(&a, 0, sizeof a);
     a.g = h->g;
     a.pz = h->pz;
     a.twz = h->twz;
     a.zscale = 1.0 / std::sqrt(2.0 * h->g.nz);
-    a.svor[0] = h->svor[0];
-    a.svor[1] = h->svor[1];
+    a.svor[0] = svor ? svor[0] : h->svor[0];
+    a.svor[1] = svor ? svor[1] : h->svor[1];
     a.scal = h->scal;
     a.mode = mode;
     a.advance_time = advance_time;
@@ -617,24 +657,53 @@ static int run_mean(ps3d_handle *h, int mode, int advance_time) {
     return 0;
 }
 
+// Whether the steps of this handle run on the semi-spectral state.
+static bool semi_steps(const ps3d_handle *h) { return h->zfuse && h->p.stepper == PS3D_STEPPER_IMPL_RK4; }
+
+// svor into the form the steps of this handle keep it in, where a caller has put the
+// mixed form there (set_vorticity, resample, set): the columns combined.
+static int ensure_semi(ps3d_handle *h) {
+    if (!semi_steps(h) || h->svor_semi) return 0;
+    for (int c = 0; c < 3; ++c)
+        HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_COMBINE, h->svor[c], h->svor[c]), h->stream));
+    h->svor_semi = true;
+    return 0;
+}
+
+// The mixed form of svor, for the host and for other grids: svor itself, or decomposed
+// into qdi (which carries data only inside the steps on svor).  The state stays as it is.
+static int mixed_svor(ps3d_handle *h, double *const **src) {
+    *src = h->svor;
+    if (!h->svor_semi) return 0;
+    for (int c = 0; c < 3; ++c)
+        HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->qdi[c]), h->stream));
+    *src = h->qdi;
+    return 0;
+}
+
 // vor2vel + the adapt-stage y pass: leaves u, v, w, xi, eta, zeta, their y
-// derivatives and z midpoints x-spectral / y-physical, svel semi-spectral, the
-// projected svor (project = true) and the Parseval sums finished into scal.
-static int inverse_adapt_stage(ps3d_handle *h, bool project) {
-    ZInvArgs z = zinv_args(h);
-    if (project) {
+// derivatives and z midpoints x-spectral / y-physical, svel semi-spectral, svor
+// projected and the Parseval sums finished into scal.
+static int inverse_adapt_stage(ps3d_handle *h) {
+    const bool semi = semi_steps(h);
+    prof_begin(h, PS3D_K_ZINV);
+    if (semi) {
+        ZStageArgs z = zstage_args(h, 1, nullptr);
+        for (int c = 0; c < 3; ++c) z.mid[c] = h->mid[c];
+        HIPCHK(launch_zstage(h->zl, ZS_START, z, h->stream));
+    } else {
+        ZInvArgs z = zinv_args(h);
         z.svor_out[0] = h->svor[0];
         z.svor_out[1] = h->svor[1];
+        for (int c = 0; c < 3; ++c) z.mid[c] = h->mid[c];
+        HIPCHK(launch_zinv(h->zl, z, h->stream));
     }
-    for (int c = 0; c < 3; ++c) z.mid[c] = h->mid[c];
-    prof_begin(h, PS3D_K_ZINV);
-    HIPCHK(launch_zinv(h->zl, z, h->stream));
     prof_end(h);
     LineArgs y = line_args(h, 1, LM_INV_Y1);
     for (int c = 0; c < 3; ++c) {
         y.in[c] = h->svel[c];
         y.out[c] = h->vel[c];
-        y.in[3 + c] = h->vor[c];
+        y.in[3 + c] = semi ? h->svor[c] : h->vor[c];
         y.out[3 + c] = h->vor[c];
         y.in[6 + c] = h->mid[c];
         y.out[6 + c] = h->mid[c];
@@ -708,25 +777,20 @@ static int products(ps3d_handle *h, int phys_in, double *const *dst, bool nn_exp
     return st;
 }
 
-// Whether RK4 stage `stage`'s tendency pass also runs the vor2vel z pass of the
-// next stage (wave kernels; PS3D_ZFUSE=0 keeps them apart, for comparison).
-static bool fuse_next(const ps3d_handle *h, int mode, int stage) {
-    return mode == ZT_RK4 && stage <= 3 && h->zl.wave != 0 && h->zfuse;
-}
-
 // One fused RK stage (impl_rk4) or cn2 iteration.  stage 1 includes adapt.
 static int fused_stage(ps3d_handle *h, int mode, int stage) {
+    const bool semi = mode == ZT_RK4 && semi_steps(h);
     int st;
     double *const *rqp = h->vel;
     if (stage == 1) {
-        if ((st = inverse_adapt_stage(h, true))) return st;
+        if ((st = inverse_adapt_stage(h))) return st;
         // the products pass goes first and also takes the velocity maxima; its output
         // goes to svel (free after the y pass), as the adapt pass still reads vel
         if ((st = products(h, 0, h->svel, true, true))) return st;
         if ((st = x_adapt(h, 0, true))) return st;
         rqp = h->svel;
     } else {
-        if (!fuse_next(h, mode, stage - 1)) {
+        if (!semi) {
             ZInvArgs z = zinv_args(h);
             prof_begin(h, PS3D_K_ZINV);
             HIPCHK(launch_zinv(h->zl, z, h->stream));
@@ -740,27 +804,31 @@ static int fused_stage(ps3d_handle *h, int mode, int stage) {
         if (st) return st;
         if ((st = products(h, 0, h->vel))) return st;
     }
-    ZTendArgs t = ztend_args(h, mode, stage, rqp);
-    if (h->cnn) {
-        // closure: net on (u, v, w, omega) at the step's first stage -> physical
-        // tendency in grad, decomposed like a physical field into mid and added to the
-        // source of every stage of the step (held fixed over the step, as the
-        // subgrid term is updated once per step; mid is free after the adapt stage)
-        if (stage == 1) {
-            HIPCHK(ps3d::cnn_apply(h->cnn, h->cnn_out, h->g.zs, h->grad[0], h->grad[1], h->grad[2], h->stream));
-            if ((st = line_fields(h, 1, LM_FWD, 3, h->grad, h->grad))) return st;
-            if ((st = line_fields(h, 0, LM_FWD, 3, h->grad, h->grad))) return st;
+    if (h->cnn && stage == 1) {
+        // closure: net on (u, v, w, omega) at the step's first stage -> physical tendency
+        // in grad, made semi-spectral and added to the source of every stage of the step
+        // (held fixed over the step, as the subgrid term is updated once per step)
+        HIPCHK(ps3d::cnn_apply(h->cnn, h->cnn_out, h->g.zs, h->grad[0], h->grad[1], h->grad[2], h->stream));
+        if ((st = line_fields(h, 1, LM_FWD, 3, h->grad, h->grad))) return st;
+        if ((st = line_fields(h, 0, LM_FWD, 3, h->grad, h->grad))) return st;
+        // the passes on svor add it decomposed (mid is free after the adapt stage)
+        if (!semi)
             for (int c = 0; c < 3; ++c)
                 HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->grad[c], h->mid[c]), h->stream));
-        }
-        for (int c = 0; c < 3; ++c) t.extra[c] = h->mid[c];
     }
-    if (fuse_next(h, mode, stage)) {
-        prof_begin(h, PS3D_K_ZTEND_ZINV);
-        HIPCHK(launch_ztend_zinv_w(h->zl.nz, h->zl.wave, h->zl.nquads, t, zinv_args(h), h->stream));
+    if (semi) {
+        ZStageArgs z = zstage_args(h, stage, rqp);
+        if (h->cnn)
+            for (int c = 0; c < 3; ++c) z.extra[c] = h->grad[c];
+        const int kind = stage == 1 ? ZS_STAGE1 : stage == 4 ? ZS_STAGE4 : ZS_STAGE23;
+        prof_begin(h, stage == 4 ? PS3D_K_ZTEND : PS3D_K_ZTEND_ZINV);
+        HIPCHK(launch_zstage(h->zl, kind, z, h->stream));
         prof_end(h);
         return 0;
     }
+    ZTendArgs t = ztend_args(h, mode, stage, rqp);
+    if (h->cnn)
+        for (int c = 0; c < 3; ++c) t.extra[c] = h->mid[c];
     prof_begin(h, PS3D_K_ZTEND);
     HIPCHK(launch_ztend(h->zl, t, h->stream));
     prof_end(h);
@@ -778,7 +846,7 @@ static int one_step(ps3d_handle *h) {
     }
     for (int s = 1; s <= 4; ++s)
         if ((st = fused_stage(h, ZT_RK4, s))) return st;
-    return run_mean(h, MEAN_ADJUST, 1);
+    return semi_steps(h) ? 0 : run_mean(h, MEAN_ADJUST, 1);   // the last semi pass restores the mean itself
 }
 
 // host <-> device copies between ps3d's (0:nz, y, x) layout and the padded columns
@@ -889,6 +957,10 @@ static ps3d_handle make_view(const ps3d_handle *h, int b) {
     v.twx = h->twx; v.twy = h->twy; v.twz = h->twz;
     v.px = h->px; v.py = h->py; v.pz = h->pz;
     v.zl = h->zl;
+    v.zfuse = h->zfuse;
+    v.svor_semi = h->svor_semi;
+    v.kxb = h->kxb;
+    v.kyb = h->kyb;
     v.TQ = h->TQ; v.QPB = h->QPB; v.nquads = h->nquads;
     v.lx = h->lx; v.ly = h->ly;
     v.lxm = h->lxm; v.lxr = h->lxr; v.lyr = h->lyr;
@@ -961,10 +1033,14 @@ int ps3d_gpu_set_vorticity(ps3d_handle *h, const double *vor) {
     int st;
     for (int c = 0; c < 3; ++c)
         if ((st = copy_in(h, h->vel[c], vor + c * hv))) return st;
-    // field_decompose_physical: fftxyp2s (y then x) + decompose
+    // field_decompose_physical: fftxyp2s (y then x) + decompose (the steps on combined
+    // columns take the horizontal transforms as they are)
     if ((st = line_fields(h, 1, LM_FWD, 3, h->vel, h->vel))) return st;
-    if ((st = line_fields(h, 0, LM_FWD, 3, h->vel, h->vel))) return st;
-    for (int c = 0; c < 3; ++c) HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->vel[c], h->svor[c]), h->stream));
+    if ((st = line_fields(h, 0, LM_FWD, 3, h->vel, h->svor))) return st;
+    h->svor_semi = semi_steps(h);
+    if (!h->svor_semi)
+        for (int c = 0; c < 3; ++c)
+            HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->svor[c]), h->stream));
     return finish_setup(h);
 }
 
@@ -972,7 +1048,8 @@ int ps3d_gpu_set_vorticity(ps3d_handle *h, const double *vor) {
 // t = 0, rolling-mean state, vor2vel and init_diffusion (utils.f90:160-184).
 static int finish_setup(ps3d_handle *h) {
     int st;
-    if ((st = run_mean(h, MEAN_CALC, 0))) return st;
+    double *const *mixed;
+    if ((st = mixed_svor(h, &mixed)) || (st = run_mean(h, MEAN_CALC, 0, mixed))) return st;
     HIPCHK(hipMemsetAsync(h->scal + SC_T, 0, sizeof(double), h->stream));
     double init[4] = {0.0, 1.0, 1.0, 0.0};   // rolling mean: sma, inew, iold, filled
     HIPCHK(hipMemcpyAsync(h->scal + SC_RM_SMA, init, sizeof init, hipMemcpyHostToDevice, h->stream));
@@ -1000,7 +1077,7 @@ int ps3d_gpu_vor2vel(ps3d_handle *h) {
     if (!h) return fail(PS3D_E_ARG, "null handle");
     if (!h->have_state) return fail(PS3D_E_STATE, "vor2vel before set_vorticity");
     int st;
-    if ((st = inverse_adapt_stage(h, true))) return st;
+    if ((st = ensure_semi(h)) || (st = inverse_adapt_stage(h))) return st;
     double *f[12];
     for (int c = 0; c < 3; ++c) {
         f[c] = h->vel[c];
@@ -1071,8 +1148,13 @@ int ps3d_gpu_step(ps3d_handle *h, double *t, double dt) {
     HIPCHK(hipMemcpyAsync(h->scal + SC_T, t, sizeof(double), hipMemcpyHostToDevice, h->stream));
     HIPCHK(hipMemcpyAsync(h->scal + SC_DT, &dt, sizeof(double), hipMemcpyHostToDevice, h->stream));
     const int mode = h->p.stepper == PS3D_STEPPER_CN2 ? ZT_CN2 : ZT_RK4;
-    ZTendArgs a = ztend_args(h, mode, 1, nullptr);
-    HIPCHK(launch_zrk(h->zl, a, h->stream));
+    const bool semi = mode == ZT_RK4 && semi_steps(h);
+    if ((st = ensure_semi(h))) return st;
+    if (semi) {
+        HIPCHK(launch_zstage(h->zl, ZS_STEP, zstage_args(h, 1, h->mid), h->stream));
+    } else {
+        HIPCHK(launch_zrk(h->zl, ztend_args(h, mode, 1, nullptr), h->stream));
+    }
     if (mode == ZT_CN2) {
         if ((st = run_mean(h, MEAN_ADJUST, 0))) return st;
         for (int it = 1; it <= 2; ++it) {
@@ -1082,7 +1164,7 @@ int ps3d_gpu_step(ps3d_handle *h, double *t, double dt) {
     } else {
         for (int s = 2; s <= 4; ++s)
             if ((st = fused_stage(h, ZT_RK4, s))) return st;
-        if ((st = run_mean(h, MEAN_ADJUST, 1))) return st;
+        if (!semi && (st = run_mean(h, MEAN_ADJUST, 1))) return st;
     }
     double sc[SC_NSCAL];
     if ((st = read_scal(h, sc))) return st;
@@ -1148,6 +1230,7 @@ int ps3d_gpu_advance_n(ps3d_handle *h, double *t, int nsteps, double *diag_serie
     if (!h || !t || nsteps < 0) return fail(PS3D_E_ARG, "invalid argument");
     if (!h->have_state) return fail(PS3D_E_STATE, "advance before set_vorticity");
     int st;
+    if ((st = ensure_semi(h))) return st;
     if ((st = ensure_diag(h, std::max(1, nsteps)))) return st;
     double zero = 0.0;
     HIPCHK(hipMemcpyAsync(h->scal + SC_T, t, sizeof(double), hipMemcpyHostToDevice, h->stream));
@@ -1174,6 +1257,7 @@ int ps3d_gpu_advance_until(ps3d_handle *h, double *t, double t_stop, int nmax, d
     if (!h->have_state) return fail(PS3D_E_STATE, "advance before set_vorticity");
     if (h->cnn) return fail(PS3D_E_UNSUPPORTED, "advance_until with a closure attached: use ps3d_gpu_advance_n");
     int st;
+    if ((st = ensure_semi(h))) return st;
     if ((st = ensure_diag(h, std::max(1, nmax)))) return st;
     // SC_STEP, SC_GATE, SC_TSTOP are consecutive slots
     const double init[3] = {0.0, 0.0, std::min(t_stop, h->p.limit)};
@@ -1197,7 +1281,11 @@ int ps3d_gpu_rk_substep(ps3d_handle *h, int stage, double dt, const double *vdis
     HIPCHK(hipMemcpyAsync(h->scal + SC_DT, &dt, sizeof(double), hipMemcpyHostToDevice, h->stream));
     ZTendArgs a = ztend_args(h, ZT_RK4, stage, nullptr);
     a.rk.vdiss = dv;
-    hipError_t e = launch_zrk(h->zl, a, h->stream);
+    hipError_t e = hipSuccess;
+    for (int c = 0; c < 3 && h->svor_semi && e == hipSuccess; ++c)   // the substep takes the mixed form
+        e = launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->svor[c]), h->stream);
+    h->svor_semi = false;
+    if (e == hipSuccess) e = launch_zrk(h->zl, a, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     (void)hipFree(dv);
     if (e != hipSuccess) return fail(PS3D_E_HIP, std::string("rk_substep: ") + hipGetErrorString(e));
@@ -1209,6 +1297,7 @@ int ps3d_gpu_profile_kernels(ps3d_handle *h, int nsteps, double *ms, int *launch
     if (!h || nsteps < 1) return fail(PS3D_E_ARG, "invalid argument");
     if (!h->have_state) return fail(PS3D_E_STATE, "profile before set_vorticity");
     int st;
+    if ((st = ensure_semi(h))) return st;
     if ((st = ensure_diag(h, nsteps))) return st;
     double zero = 0.0;
     HIPCHK(hipMemcpyAsync(h->scal + SC_STEP, &zero, sizeof(double), hipMemcpyHostToDevice, h->stream));
@@ -1243,13 +1332,14 @@ int ps3d_gpu_profile_kernels(ps3d_handle *h, int nsteps, double *ms, int *launch
         bytes[PS3D_K_YFWD] = 6.0 * vol;         // 3 R + 3 W
         // z forward + update, per stage: rk4 15, 15, 15, 9 ; cn2 12, 9, 9
         bytes[PS3D_K_ZTEND] = (cn2 ? 10.0 : 13.5) * vol;
-        // fused: stage 1..3 tendency + update without the stage result (12) and the
-        // next stage's z inverse without its svor read (6 W); stage 4 alone is 9; the
-        // z inverse left is the adapt stage's (14)
-        bytes[PS3D_K_ZTEND_ZINV] = 18.0 * vol;
-        if (!cn2 && h->zl.wave && h->zfuse) {
-            bytes[PS3D_K_ZTEND] = 9.0 * vol;
-            bytes[PS3D_K_ZINV] = 14.0 * vol;
+        if (semi_steps(h)) {
+            // the share of columns the filter passes reads r, q, p and carries qdf
+            const double b = (2.0 * h->kxb + 1.0) * (2.0 * h->kyb + 1.0) / ((double)h->g.nx * h->g.ny);
+            const double band = std::min(1.0, b);
+            // stage 1: 3 R a0, 6 W + band (3 R, 3 W); stages 2, 3 also read qdf
+            bytes[PS3D_K_ZTEND_ZINV] = (9.0 + band * (6.0 + 2 * 9.0) / 3.0) * vol;
+            bytes[PS3D_K_ZTEND] = (6.0 + band * 3.0) * vol;
+            bytes[PS3D_K_ZINV] = 12.0 * vol;
         }
         bytes[PS3D_K_YINV_ADAPT] = 21.0 * vol;  // 9 R + 12 W
         // x adapt in a step: 11 R (u, w for their x derivatives, the y derivatives,
@@ -1545,7 +1635,9 @@ int ps3d_gpu_get(ps3d_handle *h, int which, double *host) {
     const size_t hv = (size_t)h->g.nx * h->g.ny * (h->g.nz + 1);
     double *const *src = nullptr;
     switch (which) {
-        case PS3D_SVOR: src = h->svor; break;
+        case PS3D_SVOR:
+            if (const int st = mixed_svor(h, &src)) return st;
+            break;
         case PS3D_VOR: src = h->vor; break;
         case PS3D_VEL: src = h->vel; break;
         case PS3D_SVEL: src = h->svel; break;
@@ -1571,7 +1663,7 @@ int ps3d_gpu_set(ps3d_handle *h, int which, const double *host) {
     const size_t hv = (size_t)h->g.nx * h->g.ny * (h->g.nz + 1);
     double *const *dst = nullptr;
     switch (which) {
-        case PS3D_SVOR: dst = h->svor; h->have_state = true; break;
+        case PS3D_SVOR: dst = h->svor; h->have_state = true; h->svor_semi = false; break;
         case PS3D_SVORTS: dst = h->mid; break;
         default: return fail(PS3D_E_UNSUPPORTED, "field cannot be set");
     }
@@ -1718,7 +1810,11 @@ int ps3d_gpu_resample(ps3d_handle *dst, ps3d_handle *src, int which) {
     HIPCHK(hipStreamSynchronize(src->stream));
     ResampleArgs a;
     std::memset(&a, 0, sizeof a);
-    double *const *s = which == PS3D_SVOR ? src->svor : src->mid;
+    double *const *s = src->mid;
+    if (which == PS3D_SVOR) {
+        if (const int st = mixed_svor(src, &s)) return st;
+        HIPCHK(hipStreamSynchronize(src->stream));
+    }
     double *const *d = which == PS3D_SVOR ? dst->svor : dst->mid;
     for (int c = 0; c < 3; ++c) {
         a.src[c] = s[c];
@@ -1736,6 +1832,7 @@ int ps3d_gpu_resample(ps3d_handle *dst, ps3d_handle *src, int which) {
         return 0;
     }
     dst->have_state = true;
+    dst->svor_semi = false;
     return finish_setup(dst);
 }
 
@@ -1770,6 +1867,7 @@ int ps3d_gpu_set_vorticity_batch(ps3d_handle *h, int b, const double *vor) {
     int st = ps3d_gpu_set_vorticity(&v, vor);
     if (st) return st;
     h->inst_set[b] = 1;
+    h->svor_semi = semi_steps(h);   // an instance without a state is zero in either form
     h->have_state = std::all_of(h->inst_set.begin(), h->inst_set.end(), [](char c) { return c != 0; });
     h->have_phys = h->have_adapt = h->have_grad = false;
     return 0;

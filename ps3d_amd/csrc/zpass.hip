@@ -715,6 +715,255 @@ __global__ void __launch_bounds__(512) k_zinv(ZInvArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// One z pass of an RK4 step on the semi-spectral state (kernels.hpp, ZStageArgs), for
+// depths without a wave kernel: a thread holds its levels of all four members, so only
+// the transforms, the z differences and the lid values go through LDS.
+// ---------------------------------------------------------------------------
+template <int ZPT, int NZ>
+__device__ __attribute__((always_inline)) inline void zsolve(const ZStageArgs &a, const ZT<ZPT> &T, const ZLds &L,
+                                                             double (&Xi)[ZPT][4], double (&Et)[ZPT][4],
+                                                             double (&C)[ZPT][4]) {
+    const Grid &g = a.g;
+    const FftPlan &P = a.pz;
+    const double sc = a.zscale;
+    const int nz = g.nz;
+    zstore(T, a.out[5], C);
+    double E[ZPT][4], Ds[ZPT][4];
+    zdiff(T, L, g, C, E);
+    // projection (inversion.f90:41-75) and the source of w, A_y - B_x = -k2l2i (fx^2 + fy^2) D
+    // (the partner's derivative factors are this member's with the sign turned)
+#pragma unroll
+    for (int s = 0; s < ZPT; ++s) {
+        double D[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) D[m] = T.fx[m] * Et[s][m ^ 1] - T.fy[m] * Xi[s][m ^ 2];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            Ds[s][m] = -T.k2l2i * (T.fx[m] * T.fx[m] + T.fy[m] * T.fy[m]) * D[m];
+            if (!T.q00) {
+                Xi[s][m] = T.k2l2i * (T.fx[m] * E[s][m ^ 1] + T.fy[m] * D[m ^ 2]);
+                Et[s][m] = T.k2l2i * (T.fy[m] * E[s][m ^ 2] - T.fx[m] * D[m ^ 1]);
+            }
+        }
+        if (T.q00) {   // the mean flow (150-165) rides in the duplicate members 1, 2
+            Ds[s][1] = Et[s][0];
+            Ds[s][2] = Xi[s][0];
+        }
+    }
+    zstore(T, a.out[3], Xi);
+    zstore(T, a.out[4], Et);
+    if (a.mid[0]) zmid3(T, L, Xi, Et, C, a.mid[0], a.mid[1], a.mid[2]);
+    double d0[4], dn[4];
+    get_lids(T, L, Ds, d0, dn);
+    double Bs[ZPT][4], As[ZPT][4];
+    {
+        Hyp h[ZPT];
+#pragma unroll
+        for (int s = 0; s < ZPT; ++s) {
+            const int z = T.z[s];
+            h[s] = hyp_all(g, T.K, T.k2l2i, T.q00, T.has[s] ? z : 0);
+            const bool in = z > 0 && z < nz;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                if (in) Ds[s][m] = Ds[s][m] - (d0[m] * h[s].phim + dn[m] * h[s].phip);
+                Bs[s][m] = d0[m] * h[s].thetam + dn[m] * h[s].thetap;
+                E[s][m] = d0[m] * h[s].dthetam + dn[m] * h[s].dthetap;
+            }
+        }
+    }
+    zdst4<ZPT, NZ>(T, L, Ds, P, a.twz, sc);
+    // green and d/dz of the sine part (107-122)
+#pragma unroll
+    for (int s = 0; s < ZPT; ++s) {
+        const int z = T.z[s];
+        const bool in = z > 0 && z < nz;
+        const double rkz = a.rkz_sc * (double)z;
+        const double green = -1.0 / (T.k2l2 + rkz * rkz);
+        const double rkzi = in ? 1.0 / rkz : 0.0;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const double ds = Ds[s][m];
+            if (in) Ds[s][m] = green * ds;
+            As[s][m] = in ? rkz * Ds[s][m] : 0.0;
+            if (T.q00) As[s][m] = m == 1 ? -rkzi * ds : (m == 2 ? rkzi * ds : 0.0);
+        }
+    }
+    zxform2<ZPT, NZ, XK_DCT, XK_DST>(T, L, As, Ds, P, a.twz, sc);
+    // w and dw/dz (134-141); (0,0): mean flow, gamtop = Lz/2 (phip00^2 - 1/3),
+    // gambot(iz) = gamtop(nz-iz) (350-369); then u, v (169-213)
+#pragma unroll
+    for (int s = 0; s < ZPT; ++s) {
+        const int z = T.has[s] ? T.z[s] : 0;
+        const bool lid = z == 0 || z == nz;
+        double U[4], V[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            Ds[s][m] = lid || T.q00 ? 0.0 : Ds[s][m] + Bs[s][m];
+            E[s][m] = E[s][m] + As[s][m];
+        }
+        if (T.q00) {
+            double zm, zp, zm2, zp2;
+            zm_zp(g, z, zm, zp);
+            zm_zp(g, nz - z, zm2, zp2);
+            const double pt = zp / g.lz, pb = zp2 / g.lz;
+            const double gamtop = 0.5 * g.lz * (pt * pt - 1.0 / 3.0);
+            const double gambot = 0.5 * g.lz * (pb * pb - 1.0 / 3.0);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                U[m] = As[s][1] + dn[1] * gamtop - d0[1] * gambot;
+                V[m] = As[s][2] - dn[2] * gamtop + d0[2] * gambot;
+            }
+        } else {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                U[m] = T.k2l2i * (T.fx[m] * E[s][m ^ 1] + T.fy[m] * C[s][m ^ 2]);
+                V[m] = T.k2l2i * (T.fy[m] * E[s][m ^ 2] - T.fx[m] * C[s][m ^ 1]);
+            }
+        }
+        if (T.has[s])
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                if (T.store[m]) {
+                    a.out[0][T.col[m] + z] = U[m];
+                    a.out[1][T.col[m] + z] = V[m];
+                }
+    }
+    zstore(T, a.out[2], Ds);
+}
+
+// (one level per thread fits four waves per SIMD without spills)
+template <int ZPT, int NZ, int M>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ZPT == 1 && M != ZS_STEP ? 4 : 1, 8)))
+k_zstage(ZStageArgs a) {
+    const Grid &g = a.g;
+    if (gated_off(g.gate)) return;
+    const ZT<ZPT> T = make_zt<ZPT>(g, a.tb, a.TQ, a.QPB, a.nquads, (long)blockIdx.y * a.bt.vol);
+    const ZLds L = zlds(a.QPB, T.N, g.nz);
+    const FftPlan &P = a.pz;
+    const double sc = a.zscale;
+    double *scal = a.scal + (size_t)blockIdx.y * SC_NSCAL;
+    double F[3][ZPT][4];
+    if constexpr (M == ZS_START) {
+        for (int k = 0; k < 3; ++k) zload(T, a.svor[k], F[k]);
+        zsolve<ZPT, NZ>(a, T, L, F[0], F[1], F[2]);
+    } else {
+        // coefficients of the substep (impl_rk4.f90:37-53, 87-89, 212-364):
+        // q = mul (a0 + ca f t), qdf += cb f t
+        const double dt = scal[SC_DT];
+        const double f0 = T.q00 ? 1.0 : (a.tb.hou_li ? exp(a.tb.filx[T.kx] + a.tb.fily[T.ky])
+                                                     : a.tb.filx[T.kx] * a.tb.fily[T.ky]);
+        double kp = 1.0;
+        for (int i = 0; i < a.tb.nnu; ++i) kp *= T.k2l2;
+        const double ep = exp(scal[SC_DFAC] * (scal[SC_VISC] * kp));
+        const double em = 1.0 / ep, epf = ep * f0;
+        constexpr bool first = M == ZS_STAGE1 || M == ZS_STEP;
+        const double ca = M == ZS_STAGE4 ? dt / 6.0 : (first || a.stage == 2 ? 0.5 * dt : dt);
+        const double cb = first ? dt / 6.0 : dt / 3.0;
+        const double mul = M == ZS_STAGE4 || (M == ZS_STAGE23 && a.stage == 3) ? em * em : em;
+        const double f = first ? f0 : (M == ZS_STAGE4 ? epf * epf : epf);
+        if constexpr (M == ZS_STEP) {
+            double S[3][ZPT][4];
+            for (int k = 0; k < 3; ++k) {
+                zload(T, a.svor[k], F[k]);
+                zload(T, a.in[k], S[k]);
+            }
+            {   // the stored tendency is mixed
+                double lo[3][4], hi[3][4];
+                get_lids3(T, L, S[0], S[1], S[2], lo, hi);
+                zxform2<ZPT, NZ, XK_DST, XK_DST>(T, L, S[0], S[1], P, a.twz, sc);
+                zdst4<ZPT, NZ>(T, L, S[2], P, a.twz, sc);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) harmonic(T, g, S[k], lo[k], hi[k], 1.0);
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+#pragma unroll
+                for (int s = 0; s < ZPT; ++s)
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        const double a0 = F[k][s][m], sq = f * S[k][s][m];
+                        S[k][s][m] = a0 + cb * sq;
+                        F[k][s][m] = mul * (a0 + ca * sq);
+                    }
+                zstore(T, a.qdf[k], S[k]);
+            }
+        } else {
+            // quads beyond the band (per quad: their r, q, p are not read) only decay; the
+            // LDS passes run for every quad of the block
+            const bool band = T.kx <= a.kxb && T.ky <= a.kyb;
+            double R[ZPT][4], Q[ZPT][4], Pp[ZPT][4], FQ[ZPT][4], FP[ZPT][4];
+            double d0[4], d1[4], d2[4], d3[4];
+            if (band) {
+                zload(T, a.in[0], R);
+                zload(T, a.in[1], Q);
+                zload(T, a.in[2], Pp);
+            } else {
+#pragma unroll
+                for (int s = 0; s < ZPT; ++s)
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) R[s][m] = Q[s][m] = Pp[s][m] = 0.0;
+            }
+            zdiff2(T, L, g, Q, FQ, d0, d1, Pp, FP, d2, d3);
+            // 0 * KE carries a non-finite state into the columns without a tendency
+            const double nf = band ? 0.0 : 0.0 * scal[SC_KE];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                double X[ZPT][4], B[ZPT][4];
+                zload(T, M == ZS_STAGE4 && band ? a.qdf[k] : a.svor[k], F[k]);
+                if (M == ZS_STAGE23 && band) zload(T, a.qdf[k], B);
+                if (band && a.extra[0]) zload(T, a.extra[k], X);
+#pragma unroll
+                for (int s = 0; s < ZPT; ++s)
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        // dxi/dt = r_y - q_z ; deta/dt = p_z - r_x ; dzeta/dt = q_x - p_y (341-367)
+                        double t = k == 0 ? T.fy[m] * R[s][m ^ 2] - FQ[s][m]
+                                 : k == 1 ? FP[s][m] - T.fx[m] * R[s][m ^ 1]
+                                          : T.fx[m] * Q[s][m ^ 1] - T.fy[m] * Pp[s][m ^ 2];
+                        if (band && a.extra[0]) t += X[s][m];
+                        const double sq = band ? f * t : nf, a0 = F[k][s][m];
+                        B[s][m] = (M == ZS_STAGE23 && band ? B[s][m] : a0) + cb * sq;
+                        F[k][s][m] = mul * (a0 + ca * sq);
+                    }
+                if (M != ZS_STAGE4 && band) zstore(T, a.qdf[k], B);
+            }
+        }
+        if constexpr (M != ZS_STAGE4) {
+            zsolve<ZPT, NZ>(a, T, L, F[0], F[1], F[2]);
+        } else {
+            // adjust_vorticity_mean (603-619) of the (0,0) column: its mean is the trapezoid
+            // sum of the combined column (field_diagnostics.f90:584-619), and the lids' shift a
+            // shift of every level.  Every quad forms the sum, so that the barrier is the block's.
+            double mean[2] = {0.0, 0.0};
+            double *part = L.lid + T.qi * 24;   // TQ / 64 <= 8 waves per quad
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+#pragma unroll
+                for (int s = 0; s < ZPT; ++s)
+                    if (T.has[s]) mean[k] += (T.z[s] == 0 || T.z[s] == T.nz) ? 0.5 * F[k][s][0] : F[k][s][0];
+#pragma unroll
+                for (int w = 32; w >= 1; w >>= 1) mean[k] += __shfl_xor(mean[k], w, 64);
+                if ((T.tq & 63) == 0) part[2 * (T.tq >> 6) + k] = mean[k];
+            }
+            __syncthreads();
+            if (T.q00) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    double v = 0.0;
+                    for (int w = 0; w < T.TQ / 64; ++w) v += part[2 * w + k];
+                    const double d = scal[SC_INI_XI + k] - v / (double)T.nz;
+#pragma unroll
+                    for (int s = 0; s < ZPT; ++s) F[k][s][0] += d;
+                }
+                // time update t += dt in two halves (impl_rk4.f90:123,149)
+                if (T.qvalid && T.tq == 0) scal[SC_T] = (scal[SC_T] + 0.5 * dt) + 0.5 * dt;
+            }
+            for (int k = 0; k < 3; ++k) zstore(T, a.svor[k], F[k]);
+        }
+    }
+}
+
 // RK4 / cn2 update of one quad from the mixed-spectral tendency S (registers).
 template <int ZPT>
 __device__ inline void rk_update(const ZT<ZPT> &T, const RkArgs &rk, int mode, int stage, double (&S)[3][ZPT][4],
@@ -1091,6 +1340,7 @@ size_t zpass_lds_bytes(int QPB, int nz) {
 static inline int zbatch(const ZInvArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1; }
 static inline int zbatch(const ZTendArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1; }
 static inline int zbatch(const ZOpArgs &) { return 1; }
+static inline int zbatch(const ZStageArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1; }
 
 // (ZPT, nz) pairs with a compile-time FFT plan; other nz use the runtime plan.
 #define PS3D_Z_SIZES(X) X(1, 32) X(1, 48) X(1, 64) X(1, 96) X(1, 128) X(1, 192) X(1, 256) X(1, 384) \
@@ -1120,12 +1370,30 @@ static inline int zbatch(const ZOpArgs &) { return 1; }
 #define ZTRY_k_ztend(Z_, N_) else if (zl.zpt == Z_ && zl.nz == N_) { ZLAUNCH(k_ztend, Z_, N_, args, zl); done_ = true; }
 #define ZTRY_k_zop(Z_, N_) else if (zl.zpt == Z_ && zl.nz == N_) { ZLAUNCH(k_zop, Z_, N_, args, zl); done_ = true; }
 
+#define ZST_LAUNCH(Z_, N_, M_) \
+    hipLaunchKernelGGL((k_zstage<Z_, N_, M_>), dim3(zl.blocks, zbatch(args)), dim3(zl.threads), zl.lds, stream, args)
+#define ZST_KINDS(X, Z_, N_) X(Z_, N_, ZS_START) X(Z_, N_, ZS_STAGE1) X(Z_, N_, ZS_STAGE23) X(Z_, N_, ZS_STAGE4) X(Z_, N_, ZS_STEP)
+
+hipError_t launch_zstage(const ZLaunch &zl, int kind, const ZStageArgs &args, hipStream_t stream) {
+    if (zl.wave) return launch_zstage_w(zl.nz, zl.nquads, kind, args, stream);
+    bool done = false;
+#define ZST_TRY(Z_, N_, M_) else if (kind == M_ && zl.zpt == Z_ && (N_ == 0 || zl.nz == N_)) { ZST_LAUNCH(Z_, N_, M_); done = true; }
+#define ZST_SIZE(Z_, N_) ZST_KINDS(ZST_TRY, Z_, N_)
+    if (false) {}
+    PS3D_Z_SIZES(ZST_SIZE)
+    ZST_SIZE(1, 0) ZST_SIZE(2, 0) ZST_SIZE(3, 0)
+#undef ZST_SIZE
+#undef ZST_TRY
+    return done ? hipGetLastError() : hipErrorInvalidValue;
+}
+
 hipError_t configure_zpass() {
     const int lds = 160 * 1024;
     hipError_t e = hipSuccess;
 #define SETA(K) \
     if (e == hipSuccess) e = hipFuncSetAttribute((const void *)(K), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-#define ZCFG3(Z_, N_) SETA((k_zinv<Z_, N_>)) SETA((k_ztend<Z_, N_>)) SETA((k_zop<Z_, N_>))
+#define ZST_SET(Z_, N_, M_) SETA((k_zstage<Z_, N_, M_>))
+#define ZCFG3(Z_, N_) SETA((k_zinv<Z_, N_>)) SETA((k_ztend<Z_, N_>)) SETA((k_zop<Z_, N_>)) ZST_KINDS(ZST_SET, Z_, N_)
     PS3D_Z_SIZES(ZCFG3)
     ZCFG3(1, 0) ZCFG3(2, 0) ZCFG3(3, 0)
     SETA(k_zrk<1>) SETA(k_zrk<2>) SETA(k_zrk<3>)

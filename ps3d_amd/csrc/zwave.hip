@@ -546,11 +546,9 @@ template <int NZ>
 struct WOps {
     WF<NZ> a, b;
 };
-// KEEP: the next stage's input stays in registers (fused with the next vor2vel
-// pass), so every member -- also one that repeats another member's column -- forms it
-template <int NZ, bool KEEP = false>
+template <int NZ>
 __device__ __attribute__((always_inline)) inline void wrk_load(const WC &c, const RkArgs &rk, int mode, int stage, int cc, WOps<NZ> &o) {
-    if (!KEEP && !c.store) return;
+    if (!c.store) return;
     // fixed destinations (a: q, qdi or qdf; b: qdf at RK4 stages 2 and 3)
     const bool two = mode != ZT_CN2 && (stage == 2 || stage == 3);
     const double *pa = (stage == 1) ? rk.q[cc] : (two ? rk.qdi[cc] : rk.qdf[cc]);
@@ -558,12 +556,10 @@ __device__ __attribute__((always_inline)) inline void wrk_load(const WC &c, cons
     if (two) wload(c, rk.qdf[cc], o.b);
 }
 
-// The column's RK coefficients.  wrk_setup reads their inputs (the step's scalars,
-// the filter and dissipation of the column: wave-uniform) where they are used;
-// the standalone tendency kernel reads them at its top instead (wrk_inputs), so that
+// The column's RK coefficients, and their inputs (the step's scalars, the filter and
+// dissipation of the column: wave-uniform), which a kernel reads at its top so that
 // those loads overlap the column loads rather than wait, in the middle of the pass,
-// behind the operands in flight (measured: 0.396 -> 0.380 ms per step at 256^3; in
-// the fused kernel the early reads measured slower, 2.37 -> 2.42 ms).
+// behind the operands in flight (tendency pass 0.396 -> 0.380 ms per step at 256^3).
 struct WRk {
     double dt, f0, vd, em, epf;
 };
@@ -607,38 +603,9 @@ __device__ inline WRk wrk_setup_from(const WC &c, const RkArgs &rk, int mode, co
     return r;
 }
 template <int NZ>
-__device__ inline WRk wrk_setup(const WC &c, const RkArgs &rk, int mode, const ZTabs &tb) {
-    WRk r;
-    const double *sc = rk.scal + (size_t)blockIdx.y * SC_NSCAL;
-    r.dt = sc[SC_DT];
-    if (c.q00)
-        r.f0 = 1.0;
-    else if (tb.hou_li)
-        r.f0 = exp(tb.filx[c.kx] + tb.fily[c.ky]);
-    else
-        r.f0 = tb.filx[c.kx] * tb.fily[c.ky];
-    double kp = 1.0;
-    for (int i = 0; i < tb.nnu; ++i) kp *= c.k2l2;
-    const double vhdis = sc[SC_VISC] * kp;
-    if (mode == ZT_CN2) {
-        r.vd = 1.0 / (1.0 + sc[SC_DFAC] * vhdis);
-        r.em = r.epf = 0.0;
-    } else {
-        const double D = rk.vdiss ? rk.vdiss[c.colidx] : sc[SC_DFAC] * vhdis;
-        const double ep = exp(D);
-        r.em = 1.0 / ep;
-        r.epf = ep * r.f0;
-        r.vd = 0.0;
-    }
-    return r;
-}
-
-// KEEP (RK4 stages 1-3): the stage's result q -- the next stage's svor -- goes to
-// keep (every lane holds the top value) instead of memory; qdi / qdf are stored.
-template <int NZ, bool KEEP = false>
 __device__ __attribute__((always_inline)) inline void wrk_apply(const WC &c, const RkArgs &rk, int mode, int stage, int cc, const WF<NZ> &S,
-                                 const WOps<NZ> &o, const WRk &r, const ZTabs &tb, WF<NZ> *keep = nullptr) {
-    if (!KEEP && !c.store) return;
+                                 const WOps<NZ> &o, const WRk &r, const ZTabs &tb) {
+    if (!c.store) return;
     constexpr int NS = WDim<NZ>::S;
     const int l = c.lane;
     const double dt = r.dt;
@@ -666,12 +633,9 @@ __device__ __attribute__((always_inline)) inline void wrk_apply(const WC &c, con
     }
     const double dt2 = 0.5 * dt, dt3 = dt / 3.0, dt6 = dt / 6.0;
     const double em = r.em, epf = r.epf;
-    // with KEEP every lane forms the (wave-uniform) top value; lane 0 stores it
-    const bool st = c.store;
 #pragma unroll
     for (int s = 0; s <= NS; ++s) {
-        if (!KEEP && s == NS && l != 0) continue;
-        const bool mine = s < NS || l == 0;
+        if (s == NS && l != 0) continue;
         const int z = s < NS ? l + 64 * s : NZ;
         const double t = s < NS ? S.v[s % NS] : S.top;
         const double a0 = s < NS ? o.a.v[s % NS] : o.a.top;
@@ -681,26 +645,17 @@ __device__ __attribute__((always_inline)) inline void wrk_apply(const WC &c, con
             const double b0 = s < NS ? o.b.v[s % NS] : o.b.top;
             const double sq = epf * t;
             q = (stage == 2 ? em : em * em) * (a0 + (stage == 2 ? dt2 : dt) * sq);
-            if (st && mine) rk.qdf[cc][i] = b0 + dt3 * sq;
+            rk.qdf[cc][i] = b0 + dt3 * sq;
         } else if (stage == 1) {
             const double sq = r.f0 * t;
             q = (a0 + dt2 * sq) * em;
-            if (st && mine) {
-                rk.qdi[cc][i] = a0;
-                rk.qdf[cc][i] = a0 + dt6 * sq;
-            }
+            rk.qdi[cc][i] = a0;
+            rk.qdf[cc][i] = a0 + dt6 * sq;
         } else {
             const double sq = (epf * epf) * t;
             q = (em * em) * (a0 + dt6 * sq);
         }
-        if constexpr (KEEP) {
-            if (s < NS)
-                keep->v[s % NS] = q;
-            else
-                keep->top = q;
-        } else {
-            rk.q[cc][i] = q;
-        }
+        rk.q[cc][i] = q;
     }
 }
 
@@ -721,13 +676,13 @@ __device__ inline void wzero(WF<NZ> &F) {
 // spills); OCC = 1 leaves it free, except at nz <= 128, where it asks for four
 // (12-36 bytes per lane of spills, measured faster than three waves without).  Both
 // variants are built; the launch shape (and the ensemble tuner) choose.
-// The body: svor from memory, or (reg != nullptr) the three components already in
-// this wave's registers (the fused tendency + next-stage pass below).
-template <int NZ>
-__device__ __attribute__((always_inline)) inline void zinv_body(const ZInvArgs &a, const WC &c, double2 *wsm,
-                                                                const WF<NZ> *reg0, const WF<NZ> *reg1,
-                                                                const WF<NZ> *reg2, const WSeed &sd,
-                                                                const WTw<WDim<NZ>::P> &tw) {
+template <int NZ, int OCC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NZ <= 128 && OCC == 1) ? 4 : OCC, 8))) k_zinv_w(ZInvArgs a) {
+    extern __shared__ double2 wsm[];
+    if (gated_off(a.g.gate)) return;
+    const WC c = make_wc(a.g, a.tb, (long)blockIdx.y * a.bt.vol);
+    const WSeed sd = make_wseed(c, a.g);
+    const WTw<WDim<NZ>::P> tw = make_tw<WDim<NZ>::P>(a.twz, c.lane);
     constexpr int S = WDim<NZ>::S;
     const Grid g = a.g;
     double2 *ws = wsm + (size_t)c.m * WDim<NZ>::WS;
@@ -736,15 +691,9 @@ __device__ __attribute__((always_inline)) inline void zinv_body(const ZInvArgs &
     const int m1 = c.m ^ 1, m2 = c.m ^ 2;
 
     WF<NZ> Xi, Et, C, D, E;
-    if (reg0) {
-        Xi = *reg0;
-        Et = *reg1;
-        C = *reg2;
-    } else {
-        wload(c, a.svor[0], Xi);
-        wload(c, a.svor[1], Et);
-        wload(c, a.svor[2], C);
-    }
+    wload(c, a.svor[0], Xi);
+    wload(c, a.svor[1], Et);
+    wload(c, a.svor[2], C);
 
     // D = B_x - A_y (inversion.f90:41-45)
     constexpr bool DB = WDim<NZ>::DB;
@@ -932,25 +881,18 @@ __device__ __attribute__((always_inline)) inline void zinv_body(const ZInvArgs &
     }
 }
 
-template <int NZ, int OCC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NZ <= 128 && OCC == 1) ? 4 : OCC, 8))) k_zinv_w(ZInvArgs a) {
-    extern __shared__ double2 wsm[];
-    if (gated_off(a.g.gate)) return;
-    const WC c = make_wc(a.g, a.tb, (long)blockIdx.y * a.bt.vol);
-    zinv_body<NZ>(a, c, wsm, nullptr, nullptr, nullptr, make_wseed(c, a.g), make_tw<WDim<NZ>::P>(a.twz, c.lane));
-}
-
 // ---------------------------------------------------------------------------
 // vorticity_tendency, vertical part (inversion.f90:298-371), fused with one RK4
 // substep or cn2 update; one wave per member.  Same contract as k_ztend.
 // ---------------------------------------------------------------------------
-// The body; KEEP (RK4 stages 1-3): the stage's result stays in keep[3] for the
-// next stage's vor2vel pass instead of going to memory.
-template <int NZ, bool KEEP>
-__device__ __attribute__((always_inline)) inline void ztend_body(const ZTendArgs &a, const WC &c, double2 *wsm,
-                                                                 WF<NZ> *keep0, WF<NZ> *keep1, WF<NZ> *keep2,
-                                                                 const WSeed &sd,
-                                                                 const WTw<WDim<NZ>::P> &tw, const WRkIn *rin) {
+template <int NZ, int OCC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NZ <= 128 && OCC == 1) ? 4 : OCC, 8))) k_ztend_w(ZTendArgs a) {
+    extern __shared__ double2 wsm[];
+    if (gated_off(a.g.gate)) return;
+    const WC c = make_wc(a.g, a.tb, (long)blockIdx.y * a.bt.vol);
+    const WRkIn rin = wrk_inputs(c, a.rk, a.tb);
+    const WSeed sd = make_wseed(c, a.g);
+    const WTw<WDim<NZ>::P> tw = make_tw<WDim<NZ>::P>(a.twz, c.lane);
     constexpr int S = WDim<NZ>::S;
     const Grid g = a.g;
     double2 *ws = wsm + (size_t)c.m * WDim<NZ>::WS;
@@ -981,9 +923,9 @@ __device__ __attribute__((always_inline)) inline void ztend_body(const ZTendArgs
         wxform<NZ, WK_DST, WK_NONE>(c, Pp, none, ws, tw, sc);
     }
     // operands of the first component's update: in flight across the exchange
-    const bool upd = KEEP || a.mode != ZT_STORE;
+    const bool upd = a.mode != ZT_STORE;
     WOps<NZ> ops;
-    if (upd) wrk_load<NZ, KEEP>(c, a.rk, a.mode, a.stage, 0, ops);
+    if (upd) wrk_load<NZ>(c, a.rk, a.mode, a.stage, 0, ops);
     // dxi/dt = r_y - q_z ; deta/dt = p_z - r_x ; dzeta/dt = q_x - p_y (341-367)
     xput(c, wsm, 0, R);
     xput(c, wsm, 1, Q);
@@ -1021,68 +963,359 @@ __device__ __attribute__((always_inline)) inline void ztend_body(const ZTendArgs
         for (int cc = 0; cc < 3; ++cc) wstore(c, a.svorts[cc], St[cc]);
         return;
     }
-    const WRk rr = rin ? wrk_setup_from<NZ>(c, a.rk, a.mode, a.tb, *rin) : wrk_setup<NZ>(c, a.rk, a.mode, a.tb);
-    if constexpr (NZ >= 512) {
-        // nz = 512: the three components written out in sequence, the kept results in
-        // three separate variables (as one array indexed in the loop below they were
-        // kept in scratch memory, 224 bytes per lane): fused kernel 30.6 -> 28.2-29.8
-        // ms per 512^3 step (two builds with identical code for it measured both ends:
-        // its 96 KB of code exceed the instruction cache, and where the library places
-        // it matters).  At nz <= 256 the loop and the array measured as fast or faster.
-        WOps<NZ> o1, o2;
-        wrk_load<NZ, KEEP>(c, a.rk, a.mode, a.stage, 1, o1);
-        wrk_apply<NZ, KEEP>(c, a.rk, a.mode, a.stage, 0, St[0], ops, rr, a.tb, KEEP ? keep0 : nullptr);
-        wrk_load<NZ, KEEP>(c, a.rk, a.mode, a.stage, 2, o2);
-        wrk_apply<NZ, KEEP>(c, a.rk, a.mode, a.stage, 1, St[1], o1, rr, a.tb, KEEP ? keep1 : nullptr);
-        wrk_apply<NZ, KEEP>(c, a.rk, a.mode, a.stage, 2, St[2], o2, rr, a.tb, KEEP ? keep2 : nullptr);
-    } else {
+    const WRk rr = wrk_setup_from<NZ>(c, a.rk, a.mode, a.tb, rin);
 #pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-            WOps<NZ> nxt;
-            if (cc < 2) wrk_load<NZ, KEEP>(c, a.rk, a.mode, a.stage, cc + 1, nxt);
-            // (below nz = 512 the kept results are one array: keep1 = keep0 + 1, ...)
-            wrk_apply<NZ, KEEP>(c, a.rk, a.mode, a.stage, cc, St[cc], ops, rr, a.tb, KEEP ? keep0 + cc : nullptr);
-            if (cc < 2) ops = nxt;
-        }
+    for (int cc = 0; cc < 3; ++cc) {
+        WOps<NZ> nxt;
+        if (cc < 2) wrk_load<NZ>(c, a.rk, a.mode, a.stage, cc + 1, nxt);
+        wrk_apply<NZ>(c, a.rk, a.mode, a.stage, cc, St[cc], ops, rr, a.tb);
+        if (cc < 2) ops = nxt;
     }
 }
 
-template <int NZ, int OCC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NZ <= 128 && OCC == 1) ? 4 : OCC, 8))) k_ztend_w(ZTendArgs a) {
-    extern __shared__ double2 wsm[];
-    if (gated_off(a.g.gate)) return;
-    const WC c = make_wc(a.g, a.tb, (long)blockIdx.y * a.bt.vol);
-    const WRkIn rin = wrk_inputs(c, a.rk, a.tb);
-    ztend_body<NZ, false>(a, c, wsm, nullptr, nullptr, nullptr, make_wseed(c, a.g), make_tw<WDim<NZ>::P>(a.twz, c.lane),
-                          &rin);
+// ---------------------------------------------------------------------------
+// One z pass of an RK4 step on the semi-spectral state (kernels.hpp, ZStageArgs): the
+// same formulas as the two passes above, one wave per quad member.
+//
+// Two FFT calls per pass instead of seven: the DST of the source of w, then the DCT /
+// DST pair of w and dw/dz.  The source itself needs no exchange: with A, B of the
+// projection, A_y - B_x = -k2l2i (fx^2 + fy^2) D, because the partner's derivative
+// factors are this member's with the sign turned.  Two exchanges are left in the
+// vor2vel part (xi, eta, d zeta/dz together; then dw/dz and zeta), one in the tendency.
+// Measured per call at 256^3 (tendency, substep and vor2vel of the passes on svor in one
+// kernel before: 800 us): stage 1 366 us, stages 2 and 3 444 us; last stage 382 -> 232 us;
+// first pass 505 -> 421 us.  512^3: 10.1 -> 4.2 and 4.8 ms.  What bounds them now is memory:
+// 4.4 TB/s at 256^3 (stages 2, 3: 14.4 volumes) with three waves per SIMD.
+// ---------------------------------------------------------------------------
+// Region 0: the wave's FFT slice; region 1 (XB): three fields per member beside the
+// slices, where the LDS leaves room for it at full occupancy (nz <= 128): the exchange of
+// the vor2vel part then goes there and no exchange needs a barrier after its reads.
+template <int NZ>
+struct WStage {
+    static constexpr bool XB = NZ <= 128;
+    static constexpr size_t lds = 4 * (size_t)WDim<NZ>::WS * sizeof(double2) + (XB ? (size_t)12 * (NZ + 1) * sizeof(double) : 0);
+};
+template <int NZ>
+__device__ inline double *sslot(double2 *wsm, int member, int field, bool b) {
+    if (b)
+        return reinterpret_cast<double *>(wsm + (size_t)4 * WDim<NZ>::WS) + (member * 3 + field) * (NZ + 1);
+    return reinterpret_cast<double *>(wsm + (size_t)member * WDim<NZ>::WS) + field * (NZ + 1);
+}
+template <int NZ>
+__device__ inline void sput(const WC &c, double2 *wsm, int field, bool b, const WF<NZ> &F) {
+    double *p = sslot<NZ>(wsm, c.m, field, b);
+#pragma unroll
+    for (int s = 0; s < WDim<NZ>::S; ++s) p[c.lane + 64 * s] = F.v[s];
+    if (c.lane == 0) p[NZ] = F.top;
+}
+// O = c1 * (field f1 of member m1) + c2 * (field f2 of member m2)
+template <int NZ>
+__device__ inline void sget2(const WC &c, double2 *wsm, bool b, double c1, int m1, int f1, double c2, int m2, int f2,
+                             WF<NZ> &O) {
+    const double *p = sslot<NZ>(wsm, m1, f1, b), *q = sslot<NZ>(wsm, m2, f2, b);
+#pragma unroll
+    for (int s = 0; s < WDim<NZ>::S; ++s) O.v[s] = c1 * p[c.lane + 64 * s] + c2 * q[c.lane + 64 * s];
+    O.top = c1 * p[NZ] + c2 * q[NZ];
 }
 
-// RK4 stage s (1..3) of the tendency pass and the vor2vel z pass of stage s+1 in
-// one kernel: the new svor of each column never leaves the registers of the wave
-// that formed it (saves writing and re-reading three volumes per stage boundary).
-// At nz = 512 one barrier separates the two partner exchanges' uses of the block's
-// LDS.
-template <int NZ, int OCC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NZ <= 128 && OCC == 1) ? 4 : OCC, 8)))
-k_ztend_zinv_w(ZTendArgs a, ZInvArgs b) {
+// vor2vel of the combined columns Xi, Et, C of the block's four members.  free0: the
+// slices hold nothing that another wave still reads.
+template <int NZ>
+__device__ __attribute__((always_inline)) inline void wsolve(const ZStageArgs &a, const WC &c, double2 *wsm, WF<NZ> &Xi,
+                                                             WF<NZ> &Et, WF<NZ> &C, const WSeed &sd,
+                                                             const WTw<WDim<NZ>::P> &tw) {
+    constexpr int S = WDim<NZ>::S;
+    constexpr bool XB = WStage<NZ>::XB;
+    const Grid &g = a.g;
+    double2 *ws = wsm + (size_t)c.m * WDim<NZ>::WS;
+    const double sc = a.zscale;
+    const int l = c.lane, m1 = c.m ^ 1, m2 = c.m ^ 2, m3 = c.m ^ 3;
+
+    wstore(c, a.out[5], C);
+    WF<NZ> E, Ds;
+    wdiff(c, g, C, E);
+    sput(c, wsm, 0, XB, Xi);
+    sput(c, wsm, 1, XB, Et);
+    sput(c, wsm, 2, XB, E);
+    __syncthreads();
+    // D = B_x - A_y of this member and of the partners (inversion.f90:41-45); projection
+    // A = k2l2i (E_x + D_y), B = k2l2i (E_y - D_x), (0,0) column kept (56-75)
+    {
+        WF<NZ> D, P;
+        sget2<NZ>(c, wsm, XB, c.fx, m1, 1, -c.fy, m2, 0, D);
+        const double kk = -c.k2l2i * (c.fx * c.fx + c.fy * c.fy);
+#pragma unroll
+        for (int s = 0; s < S; ++s) Ds.v[s] = kk * D.v[s];
+        Ds.top = kk * D.top;
+        if (!c.q00) {
+            const WF<NZ> X0 = Xi;
+            // D of the y partner: fx eta(m3) + fy xi(m); of the x partner: -fx eta(m) - fy xi(m3)
+            sget2<NZ>(c, wsm, XB, c.fx, m1, 2, c.fy * c.fx, m3, 1, P);
+            const double fyy = c.fy * c.fy, fxx = c.fx * c.fx;
+#pragma unroll
+            for (int s = 0; s < S; ++s) Xi.v[s] = c.k2l2i * (P.v[s] + fyy * X0.v[s]);
+            Xi.top = c.k2l2i * (P.top + fyy * X0.top);
+            sget2<NZ>(c, wsm, XB, c.fy, m2, 2, c.fx * c.fy, m3, 0, P);
+#pragma unroll
+            for (int s = 0; s < S; ++s) Et.v[s] = c.k2l2i * (P.v[s] + fxx * Et.v[s]);
+            Et.top = c.k2l2i * (P.top + fxx * Et.top);
+        } else if (c.m == 1) {   // the mean flow (150-165) rides in members 1, 2 of quad (0,0)
+            Ds = Et;
+        } else if (c.m == 2) {
+            Ds = Xi;
+        }
+    }
+    if constexpr (!XB) __syncthreads();   // the slices are the FFTs' next
+    wstore(c, a.out[3], Xi);
+    wstore(c, a.out[4], Et);
+    if (a.mid[0]) {
+        WF<NZ> M;
+        wmid(c, Xi, M);
+        wstore(c, a.mid[0], M);
+        wmid(c, Et, M);
+        wstore(c, a.mid[1], M);
+        wmid(c, C, M);
+        wstore(c, a.mid[2], M);
+    }
+    // decompose the source of w (86-90)
+    const double d0 = wlo(Ds), dn = Ds.top;
+    {
+        const WPhi<NZ> ph = make_phi<NZ>(c, g, sd);
+        wharm(c, ph, Ds, d0, dn, -1.0);
+        WF<NZ> none;
+        wxform<NZ, WK_DST, WK_NONE>(c, Ds, none, ws, tw, sc);
+    }
+    // boundary parts (94-104), green and d/dz of the sine part (107-122)
+    WF<NZ> As, Bs;
+    const WExp<NZ> wx = make_wexp<NZ>(sd);
+#pragma unroll
+    for (int s = 0; s <= S; ++s) {
+        const int z = s < S ? l + 64 * s : NZ;
+        const Hyp h = hyp_from(g, c.K, c.k2l2i, c.q00, z, wx.ep[s], wx.em[s], wx.ef, wx.div);
+        const double rkz = a.rkz_sc * (double)z;
+        const double green = -1.0 / (c.k2l2 + rkz * rkz);
+        const bool interior = z > 0 && z < NZ;
+        const double dsv = s < S ? Ds.v[s % S] : Ds.top;
+        const double dg = interior ? green * dsv : dsv;
+        double as = interior ? rkz * dg : 0.0;
+        if (c.q00) {
+            const double rkzi = interior ? 1.0 / rkz : 0.0;
+            as = !interior || c.m == 0 || c.m == 3 ? 0.0 : (c.m == 1 ? -rkzi * dsv : rkzi * dsv);
+        }
+        const double bs = d0 * h.thetam + dn * h.thetap;
+        const double es = d0 * h.dthetam + dn * h.dthetap;
+        if (s < S) {
+            Bs.v[s] = bs;
+            E.v[s] = es;
+            Ds.v[s] = dg;
+            As.v[s] = as;
+        } else {
+            Bs.top = bs;
+            E.top = es;
+            Ds.top = dg;
+            As.top = as;
+        }
+    }
+    wxform<NZ, WK_DCT, WK_DST>(c, As, Ds, ws, tw, sc);
+    // w and dw/dz (134-141)
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        Ds.v[s] = l + 64 * s == 0 ? 0.0 : Ds.v[s] + Bs.v[s];
+        E.v[s] = E.v[s] + As.v[s];
+    }
+    Ds.top = 0.0;
+    E.top = E.top + As.top;
+    if (c.q00) {
+        // the mean flow: its sine part's DCT, plus gamtop = Lz/2 (phip00^2 - 1/3) and
+        // gambot(iz) = gamtop(nz-iz) (350-369); w has no (0,0) part
+#pragma unroll
+        for (int s = 0; s <= S; ++s) {
+            const int z = s < S ? l + 64 * s : NZ;
+            double zm, zp, zm2, zp2;
+            zm_zp(g, z, zm, zp);
+            zm_zp(g, NZ - z, zm2, zp2);
+            const double pt = zp / g.lz, pb = zp2 / g.lz;
+            const double gamtop = 0.5 * g.lz * (pt * pt - 1.0 / 3.0);
+            const double gambot = 0.5 * g.lz * (pb * pb - 1.0 / 3.0);
+            const double as = s < S ? As.v[s % S] : As.top;
+            const double v = c.m == 1 ? as + dn * gamtop - d0 * gambot : as - dn * gamtop + d0 * gambot;
+            if (s < S) {
+                E.v[s] = v;
+                Ds.v[s] = 0.0;
+            } else {
+                E.top = v;
+                Ds.top = 0.0;
+            }
+        }
+    }
+    wstore(c, a.out[2], Ds);
+    // u = k2l2i (es_x + cs_y), v = k2l2i (es_y - cs_x); (0,0): ubar, vbar (169-213)
+    // (the slice is this wave's own until the barrier)
+    sput(c, wsm, 0, false, E);
+    sput(c, wsm, 1, false, C);
+    __syncthreads();
+    WF<NZ> U;
+    if (c.q00) {
+        sget2<NZ>(c, wsm, false, 1.0, 1, 0, 0.0, 1, 0, U);
+        wstore(c, a.out[0], U);
+        sget2<NZ>(c, wsm, false, 1.0, 2, 0, 0.0, 2, 0, U);
+        wstore(c, a.out[1], U);
+        return;
+    }
+    sget2<NZ>(c, wsm, false, c.k2l2i * c.fx, m1, 0, c.k2l2i * c.fy, m2, 1, U);
+    wstore(c, a.out[0], U);
+    sget2<NZ>(c, wsm, false, c.k2l2i * c.fy, m2, 0, -c.k2l2i * c.fx, m1, 1, U);
+    wstore(c, a.out[1], U);
+}
+
+// calc_vorticity_mean from the combined column: the trapezoid sum
+// (field_diagnostics.f90:584-619)
+template <int NZ>
+__device__ inline double wcolmean(const WC &c, const WF<NZ> &F) {
+    double v = 0.0;
+#pragma unroll
+    for (int s = 0; s < WDim<NZ>::S; ++s) v += (c.lane + 64 * s > 0) ? F.v[s] : 0.5 * F.v[s];
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+    return (v + 0.5 * F.top) * (1.0 / (double)NZ);
+}
+
+// waves per SIMD the stage kernels are built for: as many as their registers allow
+// without spills
+constexpr int wstage_occ(int nz, int m) {
+    return nz <= 128 ? (m == ZS_STEP ? 3 : 4) : nz <= 256 ? (m == ZS_STEP ? 2 : 3) : 1;
+}
+
+template <int NZ, int M>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(wstage_occ(NZ, M), 8)))
+k_zstage_w(ZStageArgs a) {
+    constexpr int S = WDim<NZ>::S;
+    constexpr bool XB = WStage<NZ>::XB;
     extern __shared__ double2 wsm[];
     if (gated_off(a.g.gate)) return;
-    const WC c = make_wc(a.g, a.tb, (long)blockIdx.y * a.bt.vol);
-    const WSeed sd = make_wseed(c, a.g);
-    const WTw<WDim<NZ>::P> tw = make_tw<WDim<NZ>::P>(a.twz, c.lane);   // one set of roots for both passes
-    // the stage results: three separate variables at nz = 512, one array below
-    if constexpr (NZ >= 512) {
-        WF<NZ> q0, q1, q2;
-        ztend_body<NZ, true>(a, c, wsm, &q0, &q1, &q2, sd, tw, nullptr);
-        __syncthreads();   // one LDS region: the exchanges of both passes use the slices
-        zinv_body<NZ>(b, c, wsm, &q0, &q1, &q2, sd, tw);
+    const Grid &g = a.g;
+    const WC c = make_wc(g, a.tb, (long)blockIdx.y * a.bt.vol);
+    const WTw<WDim<NZ>::P> tw = make_tw<WDim<NZ>::P>(a.twz, c.lane);   // one set of roots for the whole pass
+    double2 *ws = wsm + (size_t)c.m * WDim<NZ>::WS;
+    const double sc = a.zscale;
+    const RkArgs rk = {{}, {}, {}, a.scal, nullptr};
+    WF<NZ> F[3];
+    if constexpr (M == ZS_START || M == ZS_STEP) {
+        const WSeed sd = make_wseed(c, g);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) wload(c, a.svor[k], F[k]);
+        if constexpr (M == ZS_STEP) {
+            const WRk r = wrk_setup_from<NZ>(c, rk, ZT_RK4, a.tb, wrk_inputs(c, rk, a.tb));
+            const double dt2 = 0.5 * r.dt, dt6 = r.dt / 6.0;
+            // the stored tendency is mixed
+            WF<NZ> T[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) wload(c, a.in[k], T[k]);
+            {
+                const WPhi<NZ> ph = make_phi<NZ>(c, g, sd);
+                const double x0 = wlo(T[0]), e0 = wlo(T[1]), z0 = wlo(T[2]);
+                wxform<NZ, WK_DST, WK_DST>(c, T[0], T[1], ws, tw, sc);
+                WF<NZ> none;
+                wxform<NZ, WK_DST, WK_NONE>(c, T[2], none, ws, tw, sc);
+                wharm(c, ph, T[0], x0, T[0].top, 1.0);
+                wharm(c, ph, T[1], e0, T[1].top, 1.0);
+                wharm(c, ph, T[2], z0, T[2].top, 1.0);
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                WF<NZ> Q;
+#pragma unroll
+                for (int s = 0; s <= S; ++s) {
+                    double &q = s < S ? F[k].v[s % S] : F[k].top;
+                    const double sq = r.f0 * (s < S ? T[k].v[s % S] : T[k].top);
+                    (s < S ? Q.v[s % S] : Q.top) = q + dt6 * sq;
+                    q = (q + dt2 * sq) * r.em;
+                }
+                wstore(c, a.qdf[k], Q);
+            }
+        }
+        wsolve<NZ>(a, c, wsm, F[0], F[1], F[2], sd, tw);
     } else {
-        static_assert(WDim<NZ>::DB, "second exchange region below nz = 512");
-        // (with the second region the vor2vel pass's first exchange does not touch the
-        // slices the tendency pass's exchange used)
-        WF<NZ> q[3];
-        ztend_body<NZ, true>(a, c, wsm, q, q + 1, q + 2, sd, tw, nullptr);
-        zinv_body<NZ>(b, c, wsm, q, q + 1, q + 2, sd, tw);
+        const bool band = c.kx <= a.kxb && c.ky <= a.kyb;   // block-uniform
+        const WRk r = wrk_setup_from<NZ>(c, rk, ZT_RK4, a.tb, wrk_inputs(c, rk, a.tb));
+        const double em2 = r.em * r.em;
+        // q = mul (a0 + ca f t), qdf += cb f t (impl_rk4.f90:212-364)
+        const double ca = M == ZS_STAGE4 ? r.dt / 6.0 : (M == ZS_STAGE1 || a.stage == 2 ? 0.5 * r.dt : r.dt);
+        const double mul = M == ZS_STAGE4 ? em2 : (M == ZS_STAGE1 || a.stage == 2 ? r.em : em2);
+        if (band) {
+            const double f = M == ZS_STAGE1 ? r.f0 : (M == ZS_STAGE4 ? r.epf * r.epf : r.epf);
+            const double cb = M == ZS_STAGE1 ? r.dt / 6.0 : r.dt / 3.0;
+            // dxi/dt = r_y - q_z ; deta/dt = p_z - r_x ; dzeta/dt = q_x - p_y (341-367)
+            WF<NZ> R, Q, P;
+            wload(c, a.in[1], Q);
+            wload(c, a.in[2], P);
+            wload(c, a.in[0], R);
+            sput(c, wsm, 1, false, Q);
+            sput(c, wsm, 2, false, P);
+            sput(c, wsm, 0, false, R);
+            WF<NZ> FQ, FP;
+            wdiff(c, g, Q, FQ);
+            wdiff(c, g, P, FP);
+            WF<NZ> A[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) wload(c, M == ZS_STAGE4 ? a.qdf[k] : a.svor[k], A[k]);
+            __syncthreads();
+            const double *r2 = sslot<NZ>(wsm, c.m ^ 2, 0, false), *r1 = sslot<NZ>(wsm, c.m ^ 1, 0, false);
+            const double *q1 = sslot<NZ>(wsm, c.m ^ 1, 1, false), *p2 = sslot<NZ>(wsm, c.m ^ 2, 2, false);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                WF<NZ> X, D;
+                if (a.extra[0]) wload(c, a.extra[k], X);
+                if (M == ZS_STAGE23) wload(c, a.qdf[k], D);
+#pragma unroll
+                for (int s = 0; s <= S; ++s) {
+                    const int z = s < S ? c.lane + 64 * s : NZ;
+                    double t = k == 0 ? c.fy * r2[z] - (s < S ? FQ.v[s % S] : FQ.top)
+                             : k == 1 ? (s < S ? FP.v[s % S] : FP.top) - c.fx * r1[z]
+                                      : c.fx * q1[z] - c.fy * p2[z];
+                    if (a.extra[0]) t += s < S ? X.v[s % S] : X.top;
+                    const double sq = f * t;
+                    const double a0 = s < S ? A[k].v[s % S] : A[k].top;
+                    const double b0 = M == ZS_STAGE23 ? (s < S ? D.v[s % S] : D.top) : a0;
+                    if (M != ZS_STAGE4) (s < S ? D.v[s % S] : D.top) = b0 + cb * sq;
+                    (s < S ? F[k].v[s % S] : F[k].top) = mul * (a0 + ca * sq);
+                }
+                if (M != ZS_STAGE4) wstore(c, a.qdf[k], D);
+            }
+            // one region: the next exchange writes the slots just read
+            if constexpr (!XB && M != ZS_STAGE4) __syncthreads();
+        } else {
+            // no tendency here: qdf stays a0, which is all that is kept of such a column
+            // (0 * KE carries a non-finite state into it, as the filtered products would)
+            const double nf = 0.0 * a.scal[(size_t)blockIdx.y * SC_NSCAL + SC_KE];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                wload(c, a.svor[k], F[k]);
+#pragma unroll
+                for (int s = 0; s < S; ++s) F[k].v[s] = mul * (F[k].v[s] + nf);
+                F[k].top = mul * (F[k].top + nf);
+            }
+        }
+        if constexpr (M != ZS_STAGE4) {
+            wsolve<NZ>(a, c, wsm, F[0], F[1], F[2], make_wseed(c, g), tw);
+        } else {
+            if (c.q00) {
+                // adjust_vorticity_mean (603-619): on the combined column the lids' shift is a
+                // shift of every level; and the time update t += dt in two halves
+                // (impl_rk4.f90:123,149)
+                double *scal = a.scal + (size_t)blockIdx.y * SC_NSCAL;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const double d = scal[SC_INI_XI + k] - wcolmean(c, F[k]);
+#pragma unroll
+                    for (int s = 0; s < S; ++s) F[k].v[s] += d;
+                    F[k].top += d;
+                }
+                if (threadIdx.x == 0) scal[SC_T] = (scal[SC_T] + 0.5 * r.dt) + 0.5 * r.dt;
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) wstore(c, a.svor[k], F[k]);
+        }
     }
 }
 
@@ -1162,6 +1395,10 @@ size_t zwave_lds_bytes(int nz) {
 
 hipError_t configure_zwave() {
     hipError_t e = hipSuccess;
+#define SETS(NZ_, M_)                                                                                        \
+    if (e == hipSuccess)                                                                                     \
+        e = hipFuncSetAttribute((const void *)(k_zstage_w<NZ_, M_>), hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                (int)WStage<NZ_>::lds);
 #define SETW(NZ_)                                                                                            \
     if (e == hipSuccess)                                                                                     \
         e = hipFuncSetAttribute((const void *)(k_zinv_w<NZ_, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, \
@@ -1175,17 +1412,13 @@ hipError_t configure_zwave() {
     if (e == hipSuccess)                                                                                     \
         e = hipFuncSetAttribute((const void *)(k_ztend_w<NZ_, 3>), hipFuncAttributeMaxDynamicSharedMemorySize, \
                                 (int)zwave_lds_bytes(NZ_));                                                  \
-    if (e == hipSuccess)                                                                                     \
-        e = hipFuncSetAttribute((const void *)(k_ztend_zinv_w<NZ_, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                (int)zwave_lds_bytes(NZ_));                                                  \
-    if (e == hipSuccess)                                                                                     \
-        e = hipFuncSetAttribute((const void *)(k_ztend_zinv_w<NZ_, 3>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                (int)zwave_lds_bytes(NZ_));                                                  \
+    SETS(NZ_, ZS_START) SETS(NZ_, ZS_STAGE1) SETS(NZ_, ZS_STAGE23) SETS(NZ_, ZS_STAGE4) SETS(NZ_, ZS_STEP)   \
     if (e == hipSuccess)                                                                                     \
         e = hipFuncSetAttribute((const void *)(k_zop_w<NZ_>), hipFuncAttributeMaxDynamicSharedMemorySize,    \
                                 (int)zwave_lds_bytes(NZ_));
     PS3D_ZW_SIZES(SETW)
 #undef SETW
+#undef SETS
     return e;
 }
 
@@ -1221,17 +1454,17 @@ hipError_t launch_ztend_w(int nz, int variant, int nquads, const ZTendArgs &args
     ZW_DISPATCH2(k_ztend_w, nquads, (args.bt.nb > 1 ? args.bt.nb : 1), args, variant == 1 || variant == 3);
     return hipGetLastError();
 }
-hipError_t launch_ztend_zinv_w(int nz, int variant, int nquads, const ZTendArgs &t, const ZInvArgs &z,
-                               hipStream_t stream) {
-    const int nb = t.bt.nb > 1 ? t.bt.nb : 1;
-    const bool occ3 = variant == 3;
-    switch (nz * 10 + (occ3 ? 3 : 1)) {
-#define ZTZ(NZ_, O_)                                                                                         \
-    case NZ_ * 10 + O_:                                                                                      \
-        hipLaunchKernelGGL((k_ztend_zinv_w<NZ_, O_>), dim3(nquads, nb), dim3(256), zwave_lds_bytes(NZ_), stream, t, z); \
+hipError_t launch_zstage_w(int nz, int nquads, int kind, const ZStageArgs &a, hipStream_t stream) {
+    const int nb = a.bt.nb > 1 ? a.bt.nb : 1;
+    switch (nz * 10 + kind) {
+#define ZST(NZ_, M_)                                                                                              \
+    case NZ_ * 10 + M_:                                                                                           \
+        hipLaunchKernelGGL((k_zstage_w<NZ_, M_>), dim3(nquads, nb), dim3(256), WStage<NZ_>::lds, stream, a);      \
         break;
-        ZTZ(64, 1) ZTZ(128, 1) ZTZ(256, 1) ZTZ(512, 1) ZTZ(64, 3) ZTZ(128, 3) ZTZ(256, 3) ZTZ(512, 3)
-#undef ZTZ
+#define ZSTN(NZ_) ZST(NZ_, ZS_START) ZST(NZ_, ZS_STAGE1) ZST(NZ_, ZS_STAGE23) ZST(NZ_, ZS_STAGE4) ZST(NZ_, ZS_STEP)
+        PS3D_ZW_SIZES(ZSTN)
+#undef ZSTN
+#undef ZST
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
