@@ -220,6 +220,10 @@ struct LineArgs {
     long estride;      // element stride along the line (doubles)
     long ostride;      // stride of the "other" horizontal index (doubles)
     int nother;        // number of lines in the other horizontal direction
+    // Forward passes whose result the 2/3 rule filters: slots of wavenumber index > kb are
+    // not stored, and of the other direction only the lines 0..osplit-1 and, oshift
+    // further, the rest of the nother lines are transformed (kb = n/2, osplit = nother: all).
+    int kb, osplit, oshift;
     int ZC, nzt;       // z depth of a tile, number of z tiles
     FftPlan P;
     const double2 *tw; // exp(-2 pi i m/n)

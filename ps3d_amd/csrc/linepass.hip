@@ -84,6 +84,7 @@ __device__ inline Tile make_tile(const LineArgs &a) {
     const int ti = tile_index();
     const int zt = ti % a.nzt;
     t.other = ti / a.nzt;
+    if (t.other >= a.osplit) t.other += a.oshift;
     t.z0 = zt * a.ZC;
     const int rem = a.g.nz + 1 - t.z0;
     t.zce = rem < a.ZC ? rem : a.ZC;
@@ -127,6 +128,7 @@ __device__ inline void tile_store(const Tile &t, const LineArgs &a, double *__re
         const int tot = t.n * t.nl;
         for (int e = threadIdx.x; e < tot; e += blockDim.x) {
             const int p = e % t.nl, j = e / t.nl;
+            if (j > a.kb && j < t.n - a.kb) continue;
             const double2 v = buf[(size_t)p * t.LS + t.sl(j)];
             spair(t, a, dst, j, p, make_double2(v.x * scale, v.y * scale));
         }
@@ -136,6 +138,7 @@ __device__ inline void tile_store(const Tile &t, const LineArgs &a, double *__re
     const int tot = t.n * t.ZC;
     for (int e = threadIdx.x; e < tot; e += blockDim.x) {
         const int zz = e % t.ZC, j = e / t.ZC;
+        if (j > a.kb && j < t.n - a.kb) continue;
         if (zz < t.zce) dst[t.base + (long)j * a.estride + zz] = d[((size_t)(zz >> 1) * t.LS + t.sl(j)) * 2 + (zz & 1)] * scale;
     }
 }
@@ -206,6 +209,7 @@ __device__ inline void tile_store_fwd(const Tile &t, const LineArgs &a, double *
     const int tot = t.nl * N;
     for (int e = threadIdx.x; e < tot; e += blockDim.x) {
         const int p = e % t.nl, j = e / t.nl;
+        if (j > a.kb && j < N - a.kb) continue;
         const double2 *L = R + (size_t)p * t.LS;
         const double2 zj = L[t.sl(j)], zm = L[t.sl(j == 0 ? 0 : N - j)];
         double2 v;

@@ -489,6 +489,8 @@ static LineArgs line_args(const ps3d_handle *h, int axis, int mode) {
     a.estride = c.estride;
     a.ostride = c.ostride;
     a.nother = c.nother;
+    a.kb = c.n / 2;
+    a.osplit = c.nother;
     a.ZC = c.ZC;
     a.nzt = c.nzt;
     a.P = axis == 0 ? h->px : h->py;
@@ -516,6 +518,18 @@ static int line_fields(ps3d_handle *h, int axis, int mode, int nf, double *const
         a.out[f] = out[f];
     }
     return run_line(h, a);
+}
+
+// Forward passes of fields that only the semi-spectral tendency passes read: the
+// coefficients beyond the filter's band are neither stored nor, along y, formed.
+static void band_x(const ps3d_handle *h, LineArgs &a) { a.kb = h->kxb; }
+static void band_y(const ps3d_handle *h, LineArgs &a) {
+    a.kb = h->kyb;
+    if (2 * h->kxb + 1 < h->g.nx) {
+        a.osplit = h->kxb + 1;
+        a.nother = 2 * h->kxb + 1;
+        a.oshift = h->g.nx - a.nother;
+    }
 }
 
 static FinArgs fin_args(ps3d_handle *h) {
@@ -751,9 +765,12 @@ static int x_adapt(ps3d_handle *h, int phys_in, bool velmax_given = false) {
 
 // x pass (u x omega) + y forward: r, q, p left semi-spectral in dst[]; with
 // velmax, the x pass also writes the per-wave velocity maxima into partm
-static int products(ps3d_handle *h, int phys_in, double *const *dst, bool nn_export = false, bool velmax = false) {
+// (band: the result goes to a semi-spectral tendency pass)
+static int products(ps3d_handle *h, int phys_in, double *const *dst, bool band, bool nn_export = false,
+                    bool velmax = false) {
     LineArgs x = line_args(h, 0, LM_XMAIN);
     x.phys_in = phys_in;
+    if (band) band_x(h, x);
     if (velmax) {
         x.part = h->partm;
         x.bt.part = h->b_partm;
@@ -771,8 +788,12 @@ static int products(ps3d_handle *h, int phys_in, double *const *dst, bool nn_exp
     int st = run_line(h, x);
     prof_end(h);
     if (st) return st;
+    LineArgs y = line_args(h, 1, LM_FWD);
+    y.nf = 3;
+    for (int c = 0; c < 3; ++c) y.in[c] = y.out[c] = dst[c];
+    if (band) band_y(h, y);
     prof_begin(h, PS3D_K_YFWD);
-    st = line_fields(h, 1, LM_FWD, 3, dst, dst);
+    st = run_line(h, y);
     prof_end(h);
     return st;
 }
@@ -786,7 +807,7 @@ static int fused_stage(ps3d_handle *h, int mode, int stage) {
         if ((st = inverse_adapt_stage(h))) return st;
         // the products pass goes first and also takes the velocity maxima; its output
         // goes to svel (free after the y pass), as the adapt pass still reads vel
-        if ((st = products(h, 0, h->svel, true, true))) return st;
+        if ((st = products(h, 0, h->svel, semi, true, true))) return st;
         if ((st = x_adapt(h, 0, true))) return st;
         rqp = h->svel;
     } else {
@@ -802,7 +823,7 @@ static int fused_stage(ps3d_handle *h, int mode, int stage) {
         st = line_fields(h, 1, LM_INV, 6, in, out);
         prof_end(h);
         if (st) return st;
-        if ((st = products(h, 0, h->vel))) return st;
+        if ((st = products(h, 0, h->vel, semi))) return st;
     }
     if (h->cnn && stage == 1) {
         // closure: net on (u, v, w, omega) at the step's first stage -> physical tendency
@@ -1133,7 +1154,7 @@ int ps3d_gpu_source(ps3d_handle *h) {
     int st;
     // r, q, p into grad (adapt has consumed it), then the z part into svorts (= mid)
     h->have_grad = false;
-    if ((st = products(h, 1, h->grad))) return st;
+    if ((st = products(h, 1, h->grad, false))) return st;
     ZTendArgs t = ztend_args(h, ZT_STORE, 0, h->grad);
     HIPCHK(launch_ztend(h->zl, t, h->stream));
     return 0;
@@ -1328,14 +1349,16 @@ int ps3d_gpu_profile_kernels(ps3d_handle *h, int nsteps, double *ms, int *launch
         // z inverse: 3 R + 6 W; at the adapt stage + 2 W (projected svor) + 3 W (midpoints)
         bytes[PS3D_K_ZINV] = (cn2 ? (14.0 + 2 * 9.0) / 3.0 : (14.0 + 3 * 9.0) / 4.0) * vol;
         bytes[PS3D_K_YINV] = 12.0 * vol;        // 6 R + 6 W
-        bytes[PS3D_K_XMAIN] = 9.0 * vol;        // 6 R + 3 W
-        bytes[PS3D_K_YFWD] = 6.0 * vol;         // 3 R + 3 W
+        // shares of the kx slots and of the columns that the tendency filter passes
+        const bool semi = semi_steps(h);
+        const double bx = semi ? std::min(1.0, (2.0 * h->kxb + 1.0) / h->g.nx) : 1.0;
+        const double band = semi ? bx * std::min(1.0, (2.0 * h->kyb + 1.0) / h->g.ny) : 1.0;
+        bytes[PS3D_K_XMAIN] = (6.0 + 3.0 * bx) * vol;           // 6 R + 3 W
+        bytes[PS3D_K_YFWD] = (3.0 * bx + 3.0 * band) * vol;     // 3 R + 3 W
         // z forward + update, per stage: rk4 15, 15, 15, 9 ; cn2 12, 9, 9
         bytes[PS3D_K_ZTEND] = (cn2 ? 10.0 : 13.5) * vol;
-        if (semi_steps(h)) {
-            // the share of columns the filter passes reads r, q, p and carries qdf
-            const double b = (2.0 * h->kxb + 1.0) * (2.0 * h->kyb + 1.0) / ((double)h->g.nx * h->g.ny);
-            const double band = std::min(1.0, b);
+        if (semi) {
+            // only the columns in the band read r, q, p and carry qdf
             // stage 1: 3 R a0, 6 W + band (3 R, 3 W); stages 2, 3 also read qdf
             bytes[PS3D_K_ZTEND_ZINV] = (9.0 + band * (6.0 + 2 * 9.0) / 3.0) * vol;
             bytes[PS3D_K_ZTEND] = (6.0 + band * 3.0) * vol;
