@@ -126,7 +126,10 @@ struct ZStageArgs {
     double *svor[3];          // the state at the step's start; ZS_STAGE4 writes the new one
     double *qdf[3];           // the accumulated result
     double *out[6];           // u, v, w, xi, eta, zeta; ZS_START: out[3..5] = svor (projected)
-    double *mid[3];           // ZS_START: z-midpoint vorticity, or nullptr
+    // ZS_START, for the adapt stage: the z-midpoint vorticity of the tile passes, or the
+    // Parseval sums (RY_*) of each block; nullptr: left out
+    double *mid[3];
+    double *part;
     const double *extra[3];   // optional semi-spectral tendency added to the source (closure)
     double *scal;
     Batch bt;
@@ -244,6 +247,7 @@ struct LineArgs {
     float nn_scale[6];
     int rthreads;      // register-holding modes: 1024 (standard tile), 512 (half depth) or 256 (quarter)
     int sched;         // transform-only modes: FFT schedule (LS_R8 | LS_FOLD | LS_T512 bits)
+    int lw;            // take the wave kernel of the mode (linewave.hip) where there is one
 };
 // FFT schedules of the transform-only line passes: radix-8-first plan instead of
 // radix-16-first; Hermitian pair of the inverse formed in the first radix pass; 512
@@ -260,6 +264,11 @@ size_t line_lds_bytes(int n, int ZC);
 bool line_reg_ok(int n, int T);
 int line_reg_zc(int n, int T);
 hipError_t launch_line(const LineArgs &a, int nthreads, hipStream_t stream);
+// Line passes with the lines in a wave's registers (linewave.hip)
+bool linewave_ok(int n, int mode);
+int linewave_blocks(int n, int nz);   // blocks per line set of LM_XMAIN / LM_XADAPT (a partial each)
+hipError_t configure_linewave();
+hipError_t launch_linewave(const LineArgs &a, hipStream_t stream);
 
 // Reductions: finishes the Parseval sums (after LM_INV_Y1) and the adapt step
 // (after LM_XADAPT): dt, prefactor, rolling mean, diffusion factor, diag row.

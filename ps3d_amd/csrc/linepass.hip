@@ -1079,6 +1079,7 @@ bool line_sched_ok(int n, int sched) {
 
 hipError_t launch_line(const LineArgs &a, int nthreads, hipStream_t stream) {
     (void)nthreads;
+    if (a.lw && linewave_ok(a.n, a.mode)) return launch_linewave(a, stream);
     // compile-time plans need the standard tile depth of their build
     const bool reg = a.mode == LM_INV_Y1 || a.mode == LM_XMAIN || a.mode == LM_XADAPT;
     const int rt = (a.rthreads == 512 || a.rthreads == 256) ? a.rthreads : kLineThreads;

@@ -88,6 +88,9 @@ struct ps3d_handle {
     // tile, or 512 on half of it (two blocks per CU)
     LineCfg lxm{}, lxr{}, lyr{};
     int rtm = 1024, rtx = 1024, rty = 1024;
+    // line passes with the lines in registers (linewave.hip), where a length has them;
+    // PS3D_LINE_T or PS3D_LINE_SCHED keeps the tile passes, for comparison
+    bool lw = true;
     int lsx = 0, lsy = 0;          // FFT schedules of the transform-only x and y line passes
     double visc = 0.0;
     bool have_state = false, have_phys = false, have_adapt = false;
@@ -399,11 +402,17 @@ static int init_handle(ps3d_handle *h, const ps3d_params *p, bool alloc_fields, 
         // PS3D_LINE_T="m,y,x" overrides.
         int tm = nx <= 512 ? 512 : 1024, ty = ny <= 512 ? 512 : 1024, tx = nx <= 256 ? 256 : 512;
         if (std::max(nx, ny) <= 96) tm = ty = tx = 256;
-        if (const char *ev = std::getenv("PS3D_LINE_T")) std::sscanf(ev, "%d,%d,%d", &tm, &ty, &tx);
+        if (const char *ev = std::getenv("PS3D_LINE_T")) {
+            std::sscanf(ev, "%d,%d,%d", &tm, &ty, &tx);
+            h->lw = false;
+        }
         apply_line_choice(h, tm, ty, tx);
         // FFT schedules of the transform-only passes; PS3D_LINE_SCHED="x,y" overrides
         int sx = line_sched_default(nx), sy = line_sched_default(ny);
-        if (const char *ev = std::getenv("PS3D_LINE_SCHED")) std::sscanf(ev, "%d,%d", &sx, &sy);
+        if (const char *ev = std::getenv("PS3D_LINE_SCHED")) {
+            std::sscanf(ev, "%d,%d", &sx, &sy);
+            h->lw = false;
+        }
         h->lsx = line_sched_ok(nx, sx) ? sx : line_sched_default(nx);
         h->lsy = line_sched_ok(ny, sy) ? sy : line_sched_default(ny);
     }
@@ -411,6 +420,7 @@ static int init_handle(ps3d_handle *h, const ps3d_params *p, bool alloc_fields, 
     HIPCHK(ps3d::configure_zpass());
     HIPCHK(ps3d::configure_zwave());
     HIPCHK(ps3d::configure_linepass());
+    HIPCHK(ps3d::configure_linewave());
     {   // device address of the allocation-free partials array (once per device)
         double *scr = nullptr;
         HIPCHK(ps3d::stats_scratch(h->device, &scr));
@@ -420,9 +430,10 @@ static int init_handle(ps3d_handle *h, const ps3d_params *p, bool alloc_fields, 
     // per-tile partial sums sized for the shallowest tiles (2 levels), so that any
     // block size of the adapt passes fits
     const long nzt_max = (nz + 2) / 2;
-    h->b_party = (long)h->lyr.nother * nzt_max * RY_N;
-    h->b_partx = (long)h->lxr.nother * nzt_max * RX_N;
-    h->b_partm = (long)h->lxm.nother * nzt_max * RM_N;
+    // (the wave passes: one per block of the z pass, of the x pass)
+    h->b_party = std::max((long)h->lyr.nother * nzt_max, (long)h->nquads) * RY_N;
+    h->b_partx = (long)h->lxr.nother * std::max<long>(nzt_max, linewave_blocks(nx, nz)) * RX_N;
+    h->b_partm = (long)h->lxm.nother * std::max<long>(nzt_max, linewave_blocks(nx, nz)) * RM_N;
     h->b_roll = std::max(1, p->roll_mean_win_size);
     HIPCHK(hipMalloc((void **)&h->scal, sizeof(double) * SC_NSCAL * nb));
     // clears go on the handle's stream: the stream is non-blocking, so a clear on
@@ -486,6 +497,7 @@ static LineArgs line_args(const ps3d_handle *h, int axis, int mode) {
                      : (axis == 0 ? h->lx : h->ly);
     a.rthreads = mode == LM_XMAIN ? h->rtm : mode == LM_XADAPT ? h->rtx : mode == LM_INV_Y1 ? h->rty : 256;
     a.sched = axis == 0 ? h->lsx : h->lsy;
+    a.lw = h->lw;
     a.g = h->g;
     a.axis = axis;
     a.n = c.n;
@@ -698,15 +710,24 @@ static int mixed_svor(ps3d_handle *h, double *const **src) {
     return 0;
 }
 
+// Whether the adapt stage runs on the wave line passes: the Parseval sums then come from
+// the z pass and the midpoint vorticity is formed in the x pass.
+static bool wave_adapt(const ps3d_handle *h) {
+    return h->lw && semi_steps(h) && linewave_ok(h->g.nx, LM_XADAPT) && linewave_ok(h->g.ny, LM_INV_Y1);
+}
+
 // vor2vel + the adapt-stage y pass: leaves u, v, w, xi, eta, zeta, their y
 // derivatives and z midpoints x-spectral / y-physical, svel semi-spectral, svor
 // projected and the Parseval sums finished into scal.
 static int inverse_adapt_stage(ps3d_handle *h) {
-    const bool semi = semi_steps(h);
+    const bool semi = semi_steps(h), wave = wave_adapt(h);
     prof_begin(h, PS3D_K_ZINV);
     if (semi) {
         ZStageArgs z = zstage_args(h, 1, nullptr);
-        for (int c = 0; c < 3; ++c) z.mid[c] = h->mid[c];
+        if (wave)
+            z.part = h->party;
+        else
+            for (int c = 0; c < 3; ++c) z.mid[c] = h->mid[c];
         HIPCHK(launch_zstage(h->zl, ZS_START, z, h->stream));
     } else {
         ZInvArgs z = zinv_args(h);
@@ -717,12 +738,13 @@ static int inverse_adapt_stage(ps3d_handle *h) {
     }
     prof_end(h);
     LineArgs y = line_args(h, 1, LM_INV_Y1);
+    y.lw = wave;
     for (int c = 0; c < 3; ++c) {
         y.in[c] = h->svel[c];
         y.out[c] = h->vel[c];
         y.in[3 + c] = semi ? h->svor[c] : h->vor[c];
         y.out[3 + c] = h->vor[c];
-        y.in[6 + c] = h->mid[c];
+        y.in[6 + c] = wave ? nullptr : h->mid[c];
         y.out[6 + c] = h->mid[c];
         y.out[9 + c] = h->grad[c];
     }
@@ -733,7 +755,9 @@ static int inverse_adapt_stage(ps3d_handle *h) {
     prof_end(h);
     if (st) return st;
     prof_begin(h, PS3D_K_REDUCE);
-    HIPCHK(launch_fin_y(fin_args(h), h->stream));
+    FinArgs f = fin_args(h);
+    if (wave) f.nby = h->zl.wave ? h->nquads : h->zl.blocks;
+    HIPCHK(launch_fin_y(f, h->stream));
     prof_end(h);
     return 0;
 }
@@ -741,6 +765,7 @@ static int inverse_adapt_stage(ps3d_handle *h) {
 // velmax_given: the products pass of this stage has written the velocity maxima
 static int x_adapt(ps3d_handle *h, int phys_in, bool velmax_given = false) {
     LineArgs x = line_args(h, 0, LM_XADAPT);
+    x.lw = wave_adapt(h);
     x.phys_in = phys_in;
     x.velmax_given = velmax_given;
     for (int c = 0; c < 3; ++c) {
@@ -756,9 +781,10 @@ static int x_adapt(ps3d_handle *h, int phys_in, bool velmax_given = false) {
     prof_end(h);
     if (st) return st;
     FinArgs f = fin_args(h);
+    if (x.lw) f.nbx = h->lxr.nother * linewave_blocks(h->g.nx, h->g.nz);
     if (velmax_given) {
         f.partm = h->partm;
-        f.nbm = h->lxm.nother * h->lxm.nzt;
+        f.nbm = h->lxm.nother * (h->lw && linewave_ok(h->g.nx, LM_XMAIN) ? linewave_blocks(h->g.nx, h->g.nz) : h->lxm.nzt);
     }
     prof_begin(h, PS3D_K_REDUCE);
     HIPCHK(launch_fin_x(f, h->stream));
@@ -1005,7 +1031,7 @@ static ps3d_handle make_view(const ps3d_handle *h, int b) {
     v.kxb = h->kxb;
     v.kyb = h->kyb;
     v.TQ = h->TQ; v.QPB = h->QPB; v.nquads = h->nquads;
-    v.lx = h->lx; v.ly = h->ly;
+    v.lx = h->lx; v.ly = h->ly; v.lw = h->lw;
     v.lxm = h->lxm; v.lxr = h->lxr; v.lyr = h->lyr;
     v.rtm = h->rtm; v.rtx = h->rtx; v.rty = h->rty;
     v.h_rkx = h->h_rkx;
@@ -1126,7 +1152,7 @@ int ps3d_gpu_vor2vel(ps3d_handle *h) {
         f[6 + c] = h->grad[c];
         f[9 + c] = h->mid[c];
     }
-    if ((st = line_fields(h, 0, LM_INV, 12, f, f))) return st;
+    if ((st = line_fields(h, 0, LM_INV, wave_adapt(h) ? 9 : 12, f, f))) return st;   // (12: with the midpoints)
     h->have_phys = true;
     h->have_grad = true;
     h->have_adapt = false;

@@ -791,7 +791,9 @@ __device__ __attribute__((always_inline)) inline void zsolve(const ZStageArgs &a
     }
     zxform2<ZPT, NZ, XK_DCT, XK_DST>(T, L, As, Ds, P, a.twz, sc);
     // w and dw/dz (134-141); (0,0): mean flow, gamtop = Lz/2 (phip00^2 - 1/3),
-    // gambot(iz) = gamtop(nz-iz) (350-369); then u, v (169-213)
+    // gambot(iz) = gamtop(nz-iz) (350-369); then u, v (169-213), and the Parseval sums
+    double sum[RY_N] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const double wk = (T.kx == 0 || T.kx == g.nwx ? 1.0 : 2.0) * (T.ky == 0 || T.ky == g.nwy ? 1.0 : 2.0);
 #pragma unroll
     for (int s = 0; s < ZPT; ++s) {
         const int z = T.has[s] ? T.z[s] : 0;
@@ -827,14 +829,39 @@ __device__ __attribute__((always_inline)) inline void zsolve(const ZStageArgs &a
                 if (T.store[m]) {
                     a.out[0][T.col[m] + z] = U[m];
                     a.out[1][T.col[m] + z] = V[m];
+                    const double w = (lid ? 0.5 : 1.0) * wk, x = Xi[s][m], e = Et[s][m], c = C[s][m], d = Ds[s][m];
+                    sum[RY_UU] += w * (U[m] * U[m] + V[m] * V[m] + d * d);
+                    sum[RY_WW] += w * (x * x + e * e + c * c);
+                    sum[RY_UW] += w * (U[m] * x + V[m] * e + d * c);
+                    if (T.q00) {   // the (0,0) column's trapezoid sum: the mean vorticity
+                        const double q = w * sqrt((double)g.nx * g.ny);
+                        sum[RY_MX] += q * x;
+                        sum[RY_MY] += q * e;
+                        sum[RY_MZ] += q * c;
+                    }
                 }
     }
     zstore(T, a.out[2], Ds);
+    if (a.part) {
+        double *red = L.colbuf;   // free since the last transform's barrier
+#pragma unroll
+        for (int k = 0; k < RY_N; ++k) {
+#pragma unroll
+            for (int w = 32; w >= 1; w >>= 1) sum[k] += __shfl_xor(sum[k], w, 64);
+            if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * RY_N + k] = sum[k];
+        }
+        __syncthreads();
+        if (threadIdx.x < RY_N) {
+            double v = 0.0;
+            for (int w = 0; w < (int)blockDim.x / 64; ++w) v += red[w * RY_N + threadIdx.x];
+            a.part[(size_t)blockIdx.y * a.bt.party + (size_t)blockIdx.x * RY_N + threadIdx.x] = v;
+        }
+    }
 }
 
 // (one level per thread fits four waves per SIMD without spills)
 template <int ZPT, int NZ, int M>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ZPT == 1 && M != ZS_STEP ? 4 : 1, 8)))
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ZPT > 1 || M == ZS_STEP ? 1 : M == ZS_START ? 3 : 4, 8)))
 k_zstage(ZStageArgs a) {
     const Grid &g = a.g;
     if (gated_off(g.gate)) return;

@@ -1018,9 +1018,35 @@ __device__ inline void sget2(const WC &c, double2 *wsm, bool b, double c1, int m
     O.top = c1 * p[NZ] + c2 * q[NZ];
 }
 
-// vor2vel of the combined columns Xi, Et, C of the block's four members.  free0: the
-// slices hold nothing that another wave still reads.
+// calc_vorticity_mean from the combined column: the trapezoid sum
+// (field_diagnostics.f90:584-619)
 template <int NZ>
+__device__ inline double wcolmean(const WC &c, const WF<NZ> &F) {
+    double v = 0.0;
+#pragma unroll
+    for (int s = 0; s < WDim<NZ>::S; ++s) v += (c.lane + 64 * s > 0) ? F.v[s] : 0.5 * F.v[s];
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+    return (v + 0.5 * F.top) * (1.0 / (double)NZ);
+}
+
+// This lane's share of the sums of u^2, w^2 and u w over the column, lids by half.
+template <int NZ>
+__device__ inline void wsums(const WC &c, const WF<NZ> &U, const WF<NZ> &W, double (&s)[RY_N]) {
+#pragma unroll
+    for (int i = 0; i <= WDim<NZ>::S; ++i) {
+        const bool top = i == WDim<NZ>::S;
+        const double wz = top ? (c.lane == 0 ? 0.5 : 0.0) : (c.lane + 64 * i > 0 ? 1.0 : 0.5);
+        const double u = top ? U.top : U.v[i % WDim<NZ>::S], w = top ? W.top : W.v[i % WDim<NZ>::S];
+        s[RY_UU] += wz * u * u;
+        s[RY_WW] += wz * w * w;
+        s[RY_UW] += wz * u * w;
+    }
+}
+
+// vor2vel of the combined columns Xi, Et, C of the block's four members.  SUMS: also the
+// Parseval sums of velocity and vorticity.
+template <int NZ, bool SUMS = false>
 __device__ __attribute__((always_inline)) inline void wsolve(const ZStageArgs &a, const WC &c, double2 *wsm, WF<NZ> &Xi,
                                                              WF<NZ> &Et, WF<NZ> &C, const WSeed &sd,
                                                              const WTw<WDim<NZ>::P> &tw) {
@@ -1154,36 +1180,54 @@ __device__ __attribute__((always_inline)) inline void wsolve(const ZStageArgs &a
     sput(c, wsm, 0, false, E);
     sput(c, wsm, 1, false, C);
     __syncthreads();
+    // ((0,0): members 1, 2 hold ubar, vbar)
     WF<NZ> U;
-    if (c.q00) {
+    if (c.q00)
         sget2<NZ>(c, wsm, false, 1.0, 1, 0, 0.0, 1, 0, U);
-        wstore(c, a.out[0], U);
-        sget2<NZ>(c, wsm, false, 1.0, 2, 0, 0.0, 2, 0, U);
-        wstore(c, a.out[1], U);
-        return;
-    }
-    sget2<NZ>(c, wsm, false, c.k2l2i * c.fx, m1, 0, c.k2l2i * c.fy, m2, 1, U);
+    else
+        sget2<NZ>(c, wsm, false, c.k2l2i * c.fx, m1, 0, c.k2l2i * c.fy, m2, 1, U);
     wstore(c, a.out[0], U);
-    sget2<NZ>(c, wsm, false, c.k2l2i * c.fy, m2, 0, -c.k2l2i * c.fx, m1, 1, U);
+    double sum[RY_N] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (SUMS) wsums(c, U, Xi, sum);
+    if (c.q00)
+        sget2<NZ>(c, wsm, false, 1.0, 2, 0, 0.0, 2, 0, U);
+    else
+        sget2<NZ>(c, wsm, false, c.k2l2i * c.fy, m2, 0, -c.k2l2i * c.fx, m1, 1, U);
     wstore(c, a.out[1], U);
-}
-
-// calc_vorticity_mean from the combined column: the trapezoid sum
-// (field_diagnostics.f90:584-619)
-template <int NZ>
-__device__ inline double wcolmean(const WC &c, const WF<NZ> &F) {
-    double v = 0.0;
+    if (SUMS) {
+        // Parseval (unitary transforms): every slot but the cosines of wavenumber 0 and n/2
+        // stands for two; members that repeat a column do not count
+        wsums(c, U, Et, sum);
+        wsums(c, Ds, C, sum);
+        const double wk = !c.store ? 0.0 : (c.kx == 0 || c.kx == g.nwx ? 1.0 : 2.0) * (c.ky == 0 || c.ky == g.nwy ? 1.0 : 2.0);
+        if (c.q00 && c.m == 0) {
+            const double s = (double)NZ * sqrt((double)g.nx * g.ny);
+            sum[RY_MX] = s * wcolmean(c, Xi);
+            sum[RY_MY] = s * wcolmean(c, Et);
+            sum[RY_MZ] = s * wcolmean(c, C);
+        }
+        __shared__ double red[4][RY_N];
 #pragma unroll
-    for (int s = 0; s < WDim<NZ>::S; ++s) v += (c.lane + 64 * s > 0) ? F.v[s] : 0.5 * F.v[s];
+        for (int k = 0; k < RY_N; ++k) {
+            if (k < RY_MX) {
+                sum[k] *= wk;
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    return (v + 0.5 * F.top) * (1.0 / (double)NZ);
+                for (int w = 32; w >= 1; w >>= 1) sum[k] += __shfl_xor(sum[k], w, 64);
+            }
+            if (l == 0) red[c.m][k] = sum[k];
+        }
+        __syncthreads();
+        if (threadIdx.x < RY_N)
+            a.part[(size_t)blockIdx.y * a.bt.party + (size_t)blockIdx.x * RY_N + threadIdx.x] =
+                (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+    }
 }
 
 // waves per SIMD the stage kernels are built for: as many as their registers allow
-// without spills
+// without spills (the first pass holds the vorticity to the end for the sums)
 constexpr int wstage_occ(int nz, int m) {
-    return nz <= 128 ? (m == ZS_STEP ? 3 : 4) : nz <= 256 ? (m == ZS_STEP ? 2 : 3) : 1;
+    const bool more = m == ZS_STEP || m == ZS_START;
+    return nz <= 64 ? 4 : nz <= 128 ? (more ? 3 : 4) : nz <= 256 ? (more ? 2 : 3) : (more ? 1 : 2);
 }
 
 template <int NZ, int M>
@@ -1234,7 +1278,10 @@ k_zstage_w(ZStageArgs a) {
                 wstore(c, a.qdf[k], Q);
             }
         }
-        wsolve<NZ>(a, c, wsm, F[0], F[1], F[2], sd, tw);
+        if (M == ZS_START && a.part)
+            wsolve<NZ, M == ZS_START>(a, c, wsm, F[0], F[1], F[2], sd, tw);
+        else
+            wsolve<NZ>(a, c, wsm, F[0], F[1], F[2], sd, tw);
     } else {
         const bool band = c.kx <= a.kxb && c.ky <= a.kyb;   // block-uniform
         const WRk r = wrk_setup_from<NZ>(c, rk, ZT_RK4, a.tb, wrk_inputs(c, rk, a.tb));
