@@ -15,7 +15,8 @@ BUILD = os.path.join(ROOT, "_build")
 LIBDIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(LIBDIR, "libps3d_gpu.so")
 
-SOURCES = ["zpass.hip", "zwave.hip", "linepass.hip", "linewave.hip", "closure.hip", "stats.hip", "ps3d_gpu.hip", "ncfile.cpp"]
+SOURCES = ["zpass.hip", "zwave.hip", "linepass.hip", "linewave.hip",
+           "linewave_a.hip", "linewave_b.hip", "linewave_c.hip", "linewave_d.hip", "linewave_e.hip", "closure.hip", "stats.hip", "ps3d_gpu.hip", "ncfile.cpp"]
 HEADERS = ["common.hpp", "kernels.hpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

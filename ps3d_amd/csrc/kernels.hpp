@@ -165,7 +165,7 @@ hipError_t launch_zrk(const ZLaunch &zl, const ZTendArgs &args, hipStream_t stre
 hipError_t launch_zop(const ZLaunch &zl, const ZOpArgs &args, hipStream_t stream);
 hipError_t launch_zstage(const ZLaunch &zl, int kind, const ZStageArgs &args, hipStream_t stream);
 
-// wave-per-column z kernels (zwave.hip), nz in {128, 256, 512}
+// wave-per-column z kernels (zwave.hip), nz in {64, 128, 256, 512}
 bool zwave_supported(int nz);
 size_t zwave_lds_bytes(int nz);
 hipError_t configure_zwave();
@@ -267,7 +267,6 @@ hipError_t launch_line(const LineArgs &a, int nthreads, hipStream_t stream);
 // Line passes with the lines in a wave's registers (linewave.hip)
 bool linewave_ok(int n, int mode);
 int linewave_blocks(int n, int nz);   // blocks per line set of LM_XMAIN / LM_XADAPT (a partial each)
-hipError_t configure_linewave();
 hipError_t launch_linewave(const LineArgs &a, hipStream_t stream);
 
 // Reductions: finishes the Parseval sums (after LM_INV_Y1) and the adapt step

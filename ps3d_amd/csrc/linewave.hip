@@ -1,784 +1,44 @@
-// linewave.hip -- horizontal line passes with the lines in the registers of one wave.
-//
-// A wave owns G line pairs of one line set: lane = l*G + g holds elements l + L q (q < E)
-// of the complex line g, whose real and imaginary parts are the z levels 2g and 2g+1
-// (L = n/E lanes per line, G = 64/L).  In this layout a Stockham pass of radix R | E reads
-// its butterflies from the lane's own registers, and the last pass leaves its result in the
-// same layout again, so a transform needs one exchange between two passes -- through a
-// slice of LDS that only this wave uses: no block barrier, and loads, transforms and stores
-// of different waves overlap freely.  Global accesses are 16 bytes a lane, 16 G bytes in a
-// row; waves of one block take neighbouring z ranges, so that whole 128-byte lines are used
-// by one CU.  Against the tiles in LDS of linepass.hip, a field goes through LDS four times
-// instead of eight to ten, and the index arithmetic (two thirds of the instructions there)
-// is gone: addresses are a lane offset plus constants.
-//
-// The Hermitian real form of stafft (src/fft/stafft.f90:55-58, 196-403) pairs slots k and
-// n-k: element l + L q pairs with lane L - l, register E-1-q (lane 0: E-q), one more
-// exchange ("mirror").  A derivative along the line (sta3dfft.f90:304-377) is a factor
-// +-i k on the paired coefficients.
-//
-// Measured per step against the tile passes (256^3; 128^3): y inverse 1.17 -> 1.11, 0.181 ->
-// 0.119 ms; x products 1.47 -> 1.36, 0.27 -> 0.20; y forward 0.40 -> 0.35, 0.084 -> 0.068; adapt
-// stage along y 0.93 -> 0.58, 0.18 -> 0.062, and along x 0.75 -> 0.54, 0.155 -> 0.092.  The
-// transform-only passes run at 4.4 to 5.1 TB/s (a plain copy: 5.0).
-//
-// Exchanges move real and imaginary parts one after the other through half the LDS, which
-// leaves room for four waves per SIMD.
-#include "kernels.hpp"
-#include "lfft.hpp"
+// linewave.hip -- wave line passes (linewave.hpp) of the powers of two from 64, and the
+// dispatch over all built lengths.
+#include "linewave.hpp"
 
 namespace ps3d {
 
-namespace {
+// layouts of the transform-only passes (Y) and of those that hold several fields (M)
+template <> struct LwLay<64> { using Y = Lay<64, 8, 8, 8, 1>; using M = Y; };
+template <> struct LwLay<128> { using Y = Lay<128, 16, 8, 16, 1>; using M = Lay<128, 8, 8, 4, 4>; };
+template <> struct LwLay<256> { using Y = Lay<256, 16, 16, 16, 1>; using M = Lay<256, 8, 8, 8, 4>; };
+// (8 elements per lane, one level pair per wave: the held passes are 1.5-1.7x slower)
+template <> struct LwLay<512> { using Y = Lay<512, 16, 8, 8, 8>; using M = Y; };
+#define SIZES(X) X(64) X(128) X(256) X(512)
+PS3D_LW_SET(pow2, SIZES)
 
-// Line layout: length, elements per lane, radices (R2 = 1: two passes).
-template <int N_, int E_, int R0_, int R1_, int R2_>
-struct Lay {
-    static constexpr int N = N_, E = E_, R0 = R0_, R1 = R1_, R2 = R2_;
-    static constexpr int L = N / E, G = 64 / L;
-    static constexpr int SK = R0 == 16 ? 4 : 3;     // one pad slot after every R0 elements
-    static_assert(R0 * R1 * R2 == N && (R0 == 16 || R0 == 8) && L % (1 << SK) == 0 && 64 % L == 0, "line layout");
-    static constexpr int sl(int x) { return x + (x >> SK); }
-    // line stride: slots 0..n, and the G lines a 16-lane group touches start 16/G slots apart
-    // (mod 16), so that its 8-byte accesses fall on different banks
-    static constexpr int LS0 = sl(N) + 1;
-    static constexpr int LS = LS0 + ((16 / G) - LS0 % 16 + 16) % 16;
-    // twiddle tables of the second and third pass
-    static constexpr int S1 = R0, S2 = R0 * R1;
-    static constexpr int B1 = S1 <= L ? 1 : E / R1, B2 = S2 <= L ? 1 : E / R2;
-    static constexpr int T1 = B1 * (R1 - 1) * L, T2 = R2 > 1 ? B2 * (R2 - 1) * L : 0;
-    static constexpr int LEV = 2 * G;               // z levels per wave
-};
-constexpr int kLwWaves = 4;
-
-template <class Y>
-constexpr size_t lw_lds() {
-    return sizeof(double2) * (Y::T1 + Y::T2) + sizeof(double) * kLwWaves * Y::G * Y::LS;
-}
-
-// Orders a wave's LDS accesses for the compiler (the LDS runs them in order).
-__device__ inline void lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Butterfly i = l + L b of a pass with span S: its twiddle index k = i mod S and the
-// position of its output t = 0 (output t: + t S).
-template <class Y, int S>
-__device__ inline int pass_k(int l, int b) {
-    if constexpr (S <= Y::L)
-        return l % S;
-    else
-        return l + Y::L * (b % (S / Y::L));
-}
-template <class Y, int R, int S>
-__device__ inline int pass_j(int l, int b) {
-    const int i = l + Y::L * b, k = pass_k<Y, S>(l, b);
-    return (i - k) * R + k;
-}
-
-// The tables w^(k t N / (S R)) of one block, laid out [b][t - 1][l].
-template <class Y, int R, int S, int B>
-__device__ inline void fill_tw(double2 *dst, const double2 *__restrict__ tw) {
-    for (int e = threadIdx.x; e < B * (R - 1) * Y::L; e += blockDim.x) {
-        const int l = e % Y::L, t = e / Y::L % (R - 1) + 1, b = e / (Y::L * (R - 1));
-        dst[e] = tw[pass_k<Y, S>(l, b) * t * (Y::N / (S * R))];
+static bool find_set(int n, LwSet &set) {
+    static LwSet (*const sets[])() = {lw_set_pow2, lw_set_a, lw_set_b, lw_set_c, lw_set_d, lw_set_e};
+    for (auto f : sets) {
+        set = f();
+        if (set.levels(n)) return true;
     }
+    return false;
 }
-
-struct LwCtx {
-    int l, g;
-    double *w;              // the wave's line g in LDS
-    const double2 *tw;      // twiddle tables
-};
-
-template <class Y, int R, int S, int DIR, bool LAST>
-__device__ inline void lw_pass(double2 (&x)[Y::E], const LwCtx &c, const double2 *tw) {
-    constexpr int B = Y::E / R;
-    constexpr bool SHARED = S <= Y::L;   // one set of twiddles for all butterflies of a lane
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-        double2 u[R];
-#pragma unroll
-        for (int t = 0; t < R; ++t) {
-            u[t] = x[b + t * B];
-            if (S > 1 && t > 0) {
-                const double2 w = tw[((SHARED ? 0 : b) * (R - 1) + t - 1) * Y::L + c.l];
-                u[t] = DIR < 0 ? cmul(u[t], w) : cmulc(u[t], w);
-            }
-        }
-        bfly<R>(u, DIR);
-#pragma unroll
-        for (int t = 0; t < R; ++t) x[b + t * B] = u[t];
-    }
-    if constexpr (!LAST) {
-        const int nat = Y::sl(c.l);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int b = 0; b < B; ++b) {
-                const int j = pass_j<Y, R, S>(c.l, b);
-#pragma unroll
-                for (int t = 0; t < R; ++t) {
-                    // S = 1: the R = R0 outputs share a padded group; else S is a multiple of it
-                    const int a = S == 1 ? Y::sl(j) + t : Y::sl(j) + Y::sl(t * S);
-                    c.w[a] = h ? x[b + t * B].y : x[b + t * B].x;
-                }
-            }
-            lds_order();
-#pragma unroll
-            for (int q = 0; q < Y::E; ++q) (h ? x[q].y : x[q].x) = c.w[nat + Y::sl(Y::L * q)];
-            lds_order();
-        }
-    }
-}
-
-// Unscaled complex DFT of the wave's lines, natural layout in and out.
-template <class Y, int DIR>
-__device__ inline void lw_fft(double2 (&x)[Y::E], const LwCtx &c) {
-    lw_pass<Y, Y::R0, 1, DIR, false>(x, c, nullptr);
-    lw_pass<Y, Y::R1, Y::S1, DIR, Y::R2 == 1>(x, c, c.tw);
-    if constexpr (Y::R2 > 1) lw_pass<Y, Y::R2, Y::S2, DIR, true>(x, c, c.tw + Y::T1);
-}
-
-// Part h of every element into the wave's line, and the slot of element n - k of
-// k = l + L q there (k = 0: itself) by lw_mir.
-template <class Y>
-__device__ inline void lw_put(const double2 (&x)[Y::E], const LwCtx &c, int h) {
-    const int nat = Y::sl(c.l);
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q) c.w[nat + Y::sl(Y::L * q)] = h ? x[q].y : x[q].x;
-    if (c.l == 0) c.w[Y::sl(Y::N)] = h ? x[0].y : x[0].x;   // element n is element 0
-    lds_order();
-}
-template <class Y>
-__device__ inline double lw_mir(const LwCtx &c, int q) {
-    return c.w[Y::sl(Y::L - c.l) + Y::sl(Y::L * (Y::E - 1 - q))];
-}
-
-// Hermitian real spectra of two levels -> the complex line's spectrum, times sc.
-template <class Y>
-__device__ inline void lw_herm_in(double2 (&x)[Y::E], const LwCtx &c, double sc) {
-    constexpr int H = Y::E / 2;
-    double my[Y::E];
-    lw_put<Y>(x, c, 1);
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q) my[q] = lw_mir<Y>(c, q);
-    lds_order();
-    lw_put<Y>(x, c, 0);
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q) {
-        // k < n/2: s_k + i s_(n-k); k > n/2: s_(n-k) - i s_k; k = 0, n/2: s_k
-        const double mx = lw_mir<Y>(c, q);
-        double2 z = q < H ? make_double2(x[q].x - my[q], x[q].y + mx) : make_double2(mx + x[q].y, my[q] - x[q].x);
-        if ((q == 0 || q == H) && c.l == 0) z = x[q];
-        x[q] = make_double2(sc * z.x, sc * z.y);
-    }
-    lds_order();
-}
-
-// Complex spectrum -> Hermitian real spectra of the two levels, times sc.
-template <class Y>
-__device__ inline void lw_herm_out(double2 (&x)[Y::E], const LwCtx &c, double sc) {
-    constexpr int H = Y::E / 2;
-    double my[Y::E];
-    lw_put<Y>(x, c, 1);
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q) my[q] = lw_mir<Y>(c, q);
-    lds_order();
-    lw_put<Y>(x, c, 0);
-    sc *= 0.5;
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q) {
-        const double mx = lw_mir<Y>(c, q);
-        double2 lo = make_double2(x[q].x + mx, x[q].y + my[q]);
-        const double2 hi = make_double2(my[q] - x[q].y, x[q].x - mx);
-        if (q > H || (q == H && c.l > 0)) lo = hi;
-        x[q] = make_double2(sc * lo.x, sc * lo.y);
-    }
-    lds_order();
-}
-
-// Tile of a wave: z range, line set, addresses.
-template <class Y>
-struct LwTile {
-    int l, g, z0, other, tile;
-    bool any, full;         // the wave has levels; all of them (else lanes are masked)
-    bool v0, v1;            // this lane's levels exist
-    long base;              // wave-uniform element offset of (line element 0, level z0)
-    unsigned lane;          // lane's element offset
-    long estep;             // element offset of L line elements
-};
-template <class Y>
-__device__ inline LwTile<Y> lw_tile(const LineArgs &a) {
-    LwTile<Y> t;
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    t.l = lane / Y::G;
-    t.g = lane % Y::G;
-    // XCD-contiguous tile ranges, as linepass.hip's tile_index
-    const int B = gridDim.x, i = blockIdx.x, qn = B >> 3, r = B & 7, xc = i & 7, k = i >> 3;
-    t.tile = xc < r ? xc * (qn + 1) + k : r * (qn + 1) + (xc - r) * qn + k;
-    const int nz1 = a.g.nz + 1;
-    t.z0 = ((t.tile % a.nzt) * kLwWaves + wv) * Y::LEV;
-    t.other = t.tile / a.nzt;
-    if (t.other >= a.osplit) t.other += a.oshift;
-    t.any = t.z0 < nz1;
-    t.full = t.z0 + Y::LEV <= nz1;
-    t.v0 = t.z0 + 2 * t.g < nz1;
-    t.v1 = t.z0 + 2 * t.g + 1 < nz1;
-    t.base = (long)blockIdx.y * a.bt.vol + (long)t.other * a.ostride + t.z0;
-    t.lane = (unsigned)(t.l * a.estride + 2 * t.g);
-    t.estep = (long)Y::L * a.estride;
-    return t;
-}
-template <class Y>
-__device__ inline void lw_load(const LwTile<Y> &t, const double *__restrict__ src, double2 (&x)[Y::E]) {
-    const double *p = src + t.base;
-    if (t.full) {
-#pragma unroll
-        for (int q = 0; q < Y::E; ++q, p += t.estep) x[q] = *reinterpret_cast<const double2 *>(p + t.lane);
-    } else {
-        // a pair whose second level is beyond the lid reads the column's padding (16-level
-        // columns); the level is zeroed, as it shares a complex line
-#pragma unroll
-        for (int q = 0; q < Y::E; ++q, p += t.estep) {
-            x[q] = make_double2(0.0, 0.0);
-            if (t.v0) x[q] = *reinterpret_cast<const double2 *>(p + t.lane);
-            if (!t.v1) x[q].y = 0.0;
-        }
-    }
-}
-// KB: only slots of wavenumber index <= kb
-template <class Y, bool KB>
-__device__ inline void lw_store(const LwTile<Y> &t, double *__restrict__ dst, const double2 (&x)[Y::E], int kb) {
-    double *p = dst + t.base;
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q, p += t.estep) {
-        bool on = t.full || t.v0;
-        if (KB) {
-            const int j = t.l + Y::L * q;
-            on = on && (j <= kb || j >= Y::N - kb);
-        }
-        if (!on) continue;
-        if (t.full || t.v1)
-            *reinterpret_cast<double2 *>(p + t.lane) = x[q];
-        else
-            p[t.lane] = x[q].x;
-    }
-}
-
-template <class Y>
-__device__ inline LwCtx lw_ctx(const LwTile<Y> &t, double2 *smem, const LineArgs &a) {
-    LwCtx c;
-    c.l = t.l;
-    c.g = t.g;
-    c.tw = smem;
-    double *w = reinterpret_cast<double *>(smem + Y::T1 + Y::T2);
-    c.w = w + ((threadIdx.x >> 6) * Y::G + t.g) * Y::LS;
-    fill_tw<Y, Y::R1, Y::S1, Y::B1>(smem, a.tw);
-    if constexpr (Y::R2 > 1) fill_tw<Y, Y::R2, Y::S2, Y::B2>(smem + Y::T1, a.tw);
-    __syncthreads();   // the only one: the tables are read by every wave
-    return c;
-}
-
-// nf fields forward (FWD) or inverse, one per block (blockIdx.z): a wave that loops over
-// the fields leaves the last round of waves nearly empty (256^3: 8.3 waves per SIMD; 1.47
-// against 1.11 ms per step).  Three waves per SIMD: at four the 16 elements per lane spill
-// (1.16 ms).
-template <class Y, bool FWD>
-__global__ void __launch_bounds__(64 * kLwWaves) __attribute__((amdgpu_waves_per_eu(3, 8)))
-k_lw_lines(LineArgs a) {
-    extern __shared__ double2 lwsm[];
-    if (gated_off(a.g.gate)) return;
-    const LwTile<Y> t = lw_tile<Y>(a);
-    const LwCtx c = lw_ctx<Y>(t, lwsm, a);
-    if (!t.any) return;
-    const double sc = 1.0 / sqrt((double)Y::N);
-    const int f = blockIdx.z;
-    double2 x[Y::E];
-    lw_load<Y>(t, a.in[f], x);
-    if constexpr (FWD) {
-        lw_fft<Y, -1>(x, c);
-        lw_herm_out<Y>(x, c, sc);
-        lw_store<Y, true>(t, a.out[f], x, a.kb);
-    } else {
-        lw_herm_in<Y>(x, c, sc);
-        lw_fft<Y, +1>(x, c);
-        lw_store<Y, false>(t, a.out[f], x, 0);
-    }
-}
-
-// closure input: channel ch of the bf16 tensor [p][16], p = (ix*ny + iy)*(nz+1) + iz
-template <class Y>
-__device__ inline void lw_export(const LwTile<Y> &t, const LineArgs &a, const double2 (&x)[Y::E], int ch) {
-    if (!a.nn_in) return;
-    const float s = a.nn_scale[ch];
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (!(h ? t.v1 : t.v0)) continue;
-            const long p = ((long)(t.l + Y::L * q) * a.g.ny + t.other) * (a.g.nz + 1) + t.z0 + 2 * t.g + h;
-            uint32_t u = __builtin_bit_cast(uint32_t, (float)(h ? x[q].y : x[q].x) * s);
-            u += 0x7fffu + ((u >> 16) & 1u);
-            a.nn_in[p * 16 + ch] = (uint16_t)(u >> 16);
-        }
-}
-
-// Coefficients of element k times i k (derivative along the line), zero at 0 and n/2.
-template <class Y>
-__device__ inline void lw_deriv(double2 (&x)[Y::E], const LwTile<Y> &t, const double *__restrict__ rk) {
-    constexpr int H = Y::E / 2;
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q) {
-        double r = rk[t.l + Y::L * q];
-        if ((q == 0 || q == H) && t.l == 0) r = 0.0;
-        if (q >= H) r = -r;
-        x[q] = make_double2(-r * x[q].y, r * x[q].x);
-    }
-}
-
-// Adapt stage along y: nf fields inverse and, of the first three, the inverse of the
-// derivative too (out[9 + f]); the second reading of a tile comes from the caches.
-template <class Y>
-__global__ void __launch_bounds__(64 * kLwWaves) __attribute__((amdgpu_waves_per_eu(3, 8))) k_lw_inv_d(LineArgs a) {
-    extern __shared__ double2 lwsm[];
-    if (gated_off(a.g.gate)) return;
-    const LwTile<Y> t = lw_tile<Y>(a);
-    const LwCtx c = lw_ctx<Y>(t, lwsm, a);
-    if (!t.any) return;
-    const double sc = 1.0 / sqrt((double)Y::N);
-    const int f = blockIdx.z;
-    for (int d = f < 3 ? 1 : 0; d >= 0; --d) {
-        double2 x[Y::E];
-        lw_load<Y>(t, a.in[f], x);
-        lw_herm_in<Y>(x, c, sc);
-        if (d) lw_deriv<Y>(x, t, a.rk);
-        lw_fft<Y, +1>(x, c);
-        lw_store<Y, false>(t, a.out[d ? 9 + f : f], x, 0);
-    }
-}
-
-template <class Y>
-__device__ inline double lw_max(const LwTile<Y> &t, const double2 (&x)[Y::E]) {
-    double m = -INFINITY;
-#pragma unroll
-    for (int q = 0; q < Y::E; ++q) {
-        if (t.v0) m = fmax(m, x[q].x);
-        if (t.v1) m = fmax(m, x[q].y);
-    }
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) m = fmax(m, __shfl_xor(m, s));
-    return m;
-}
-
-// x products pass: r = u eta - v xi, q = w xi - u zeta, p = v zeta - w eta with
-// omega + f_cor (inversion.f90:316-352).  The fields come in the order u, eta, w, xi, v,
-// zeta, around the cycle of the six products, so that at most five are held while the sixth
-// is transformed: 250 VGPRs at eight elements per lane, two waves per SIMD.  (Measured:
-// loading each field during the transform before it spills 30 registers and is slower,
-// 1.47 against 1.36 ms per 256^3 step.)
-template <class Y>
-__global__ void __launch_bounds__(64 * kLwWaves) __attribute__((amdgpu_waves_per_eu(Y::E > 8 ? 1 : 2, 8)))
-k_lw_xmain(LineArgs a) {
-    constexpr int E = Y::E;
-    extern __shared__ double2 lwsm[];
-    if (gated_off(a.g.gate)) return;
-    const LwTile<Y> t = lw_tile<Y>(a);
-    const LwCtx c = lw_ctx<Y>(t, lwsm, a);
-    const double sc = 1.0 / sqrt((double)Y::N);
-    const bool pm = a.part != nullptr;
-    __shared__ double red[kLwWaves][RM_N];
-    auto put_max = [&](double um, double vm, double wm) {   // adapt stage: signed maxima (advance.f90:319-321)
-        if (!pm) return;
-        if ((threadIdx.x & 63) == 0) {
-            red[threadIdx.x >> 6][RM_UMAX] = um;
-            red[threadIdx.x >> 6][RM_VMAX] = vm;
-            red[threadIdx.x >> 6][RM_WMAX] = wm;
-        }
-        __syncthreads();
-        if (threadIdx.x < RM_N) {
-            double v = red[0][threadIdx.x];
-#pragma unroll
-            for (int w = 1; w < kLwWaves; ++w) v = fmax(v, red[w][threadIdx.x]);
-            a.part[(size_t)blockIdx.y * a.bt.part + (size_t)t.tile * RM_N + threadIdx.x] = v;
-        }
-    };
-    if (!t.any) {
-        put_max(-INFINITY, -INFINITY, -INFINITY);
-        return;
-    }
-    auto load = [&](int f, double2(&x)[E]) {
-        lw_load<Y>(t, a.in[f], x);
-    };
-    auto inv = [&](double2(&x)[E], int ch) {
-        if (!a.phys_in) {
-            lw_herm_in<Y>(x, c, sc);
-            lw_fft<Y, +1>(x, c);
-        }
-        lw_export<Y>(t, a, x, ch);
-    };
-    auto fwd = [&](double2(&x)[E], int f) {
-        lw_fft<Y, -1>(x, c);
-        lw_herm_out<Y>(x, c, sc);
-        lw_store<Y, true>(t, a.out[f], x, a.kb);
-    };
-    auto add = [&](double2(&x)[E], double f) {
-#pragma unroll
-        for (int i = 0; i < E; ++i) x[i] = make_double2(x[i].x + f, x[i].y + f);
-    };
-    double2 u[E], r[E], p[E], q[E], s[E], v[E];
-    load(0, u);
-    inv(u, 0);
-    const double um = pm ? lw_max<Y>(t, u) : 0.0;
-    load(4, s);
-    inv(s, 4);            // eta
-    add(s, a.fcor[1]);
-#pragma unroll
-    for (int i = 0; i < E; ++i) r[i] = make_double2(u[i].x * s[i].x, u[i].y * s[i].y);
-    load(2, v);
-    inv(v, 2);            // w
-    const double wm = pm ? lw_max<Y>(t, v) : 0.0;
-#pragma unroll
-    for (int i = 0; i < E; ++i) p[i] = make_double2(-v[i].x * s[i].x, -v[i].y * s[i].y);
-    load(3, q);
-    inv(q, 3);            // xi
-    add(q, a.fcor[0]);
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-        const double2 xi = q[i];
-        q[i] = make_double2(v[i].x * xi.x, v[i].y * xi.y);
-        v[i] = xi;
-    }
-    load(1, s);
-    inv(s, 1);            // v
-    const double vm = pm ? lw_max<Y>(t, s) : 0.0;
-#pragma unroll
-    for (int i = 0; i < E; ++i) r[i] = make_double2(r[i].x - s[i].x * v[i].x, r[i].y - s[i].y * v[i].y);
-    fwd(r, 0);
-    load(5, v);
-    inv(v, 5);            // zeta
-    add(v, a.fcor[2]);
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-        p[i] = make_double2(s[i].x * v[i].x + p[i].x, s[i].y * v[i].y + p[i].y);
-        q[i] = make_double2(q[i].x - u[i].x * v[i].x, q[i].y - u[i].y * v[i].y);
-    }
-    fwd(q, 1);
-    fwd(p, 2);
-    put_max(um, vm, wm);
-}
-
-// Largest |eigenvalue| of a traceless symmetric matrix from p^2 = tr(S^2)/6 and its
-// determinant.  The roots of the characteristic cubic are 2 p cos((acos r + 2 pi j) / 3) with
-// r = det / (2 p^3) (Smith, CACM 4(4), 1961); the largest in modulus is 2 p y with
-// 4 y^3 - 3 y = |r|, y in [sqrt(3)/2, 1]: a simple root with derivative 12 y^2 - 3 >= 6, so
-// Newton's iteration gives it to rounding.  Three steps in 32 bits, two with 64-bit
-// residuals and the 32-bit slope (error 1e-7, then 1e-14, then rounding).
-__device__ inline double eig_absmax0(double p2, double det) {
-    if (!(p2 > 0.0)) return 0.0;
-    const double p = sqrt(p2);
-    const double r = fmin(1.0, 0.5 * fabs(det) / (p2 * p));
-    const float rf = (float)r;
-    float yf = 0.8660254f + 0.1339746f * rf;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const float y2 = yf * yf;
-        yf -= (yf * (4.0f * y2 - 3.0f) - rf) * __builtin_amdgcn_rcpf(12.0f * y2 - 3.0f);
-    }
-    double y = (double)yf;
-    const double s = (double)__builtin_amdgcn_rcpf(12.0f * yf * yf - 3.0f);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) y -= (y * (4.0 * y * y - 3.0) - r) * s;
-    return 2.0 * p * y;
-}
-
-// x adapt pass (advance.f90:171-289): max |omega|, the largest |eigenvalue| of the
-// symmetrised strain, its lid maxima, and the sums of the characteristic vorticity; velocity
-// maxima where the products pass has not taken them.  S11 = u_x, S12 = u_y + zeta/2,
-// S13 = w_x + eta/2, S22 = v_y, S23 = w_y - xi/2, S33 = -(u_x + v_y) (225-257): the vorticity
-// comes first and the strain is built in its place, so that five fields are held at most.
-// The z-midpoint vorticity (field_diagnostics.f90:501-545) is formed here, from the level
-// below the wave's tile as one more line pair, instead of going through the z and y passes
-// as three more fields.  Eigenvalues lie between sqrt(3) p and 2 p, so only points with
-// p^2 >= 3/4 of the wave's largest are evaluated.
-template <class Y>
-__global__ void __launch_bounds__(64 * kLwWaves) __attribute__((amdgpu_waves_per_eu(Y::E > 8 ? 1 : 2, 8)))
-k_lw_xadapt(LineArgs a) {
-    constexpr int E = Y::E;
-    extern __shared__ double2 lwsm[];
-    if (gated_off(a.g.gate)) return;
-    const LwTile<Y> t = lw_tile<Y>(a);
-    const LwCtx c = lw_ctx<Y>(t, lwsm, a);
-    const double sc = 1.0 / sqrt((double)Y::N);
-    const int nz = a.g.nz;
-    double res[RX_N] = {0.0, 2.220446049250313e-16, 0.0, 0.0, -INFINITY, -INFINITY, -INFINITY, 0.0, 0.0};
-    if (t.any) {
-        auto inv = [&](double2(&x)[E]) {
-            if (a.phys_in) return;
-            lw_herm_in<Y>(x, c, sc);
-            lw_fft<Y, +1>(x, c);
-        };
-        auto load = [&](int f, double2(&x)[E]) {
-            lw_load<Y>(t, a.in[f], x);
-        };
-        auto deriv = [&](double2(&x)[E]) {
-            if (a.phys_in)
-                lw_fft<Y, -1>(x, c);   // the complex line's spectrum as it is
-            else
-                lw_herm_in<Y>(x, c, sc);
-            lw_deriv<Y>(x, t, a.rk);
-            lw_fft<Y, +1>(x, c);
-            if (a.phys_in)
-#pragma unroll
-                for (int q = 0; q < E; ++q) x[q] = make_double2(x[q].x * (1.0 / Y::N), x[q].y * (1.0 / Y::N));
-        };
-        double2 s1[E], s2[E], s3[E], s4[E], s5[E];
-        if (!a.velmax_given) {
-            for (int f = 0; f < 3; ++f) {
-                load(f, s1);
-                inv(s1);
-                res[RX_UMAX + f] = lw_max<Y>(t, s1);
-            }
-        }
-        load(3, s1);
-        inv(s1);    // xi
-        load(4, s2);
-        inv(s2);    // eta
-        {
-            // the level below: (xi, eta) in the first line, zeta in the second (the halo
-            // values then sit in lanes g = 0 and 1); one line per wave: two calls
-            double2 hx[E], hz[Y::G == 1 ? E : 1];
-            const long zb = t.base - 1 + (long)t.l * a.estride;
-#pragma unroll
-            for (int q = 0; q < E; ++q) {
-                hx[q] = make_double2(0.0, 0.0);
-                if (t.z0 > 0 && t.g == 0)
-                    hx[q] = make_double2(a.in[3][zb + q * t.estep], a.in[4][zb + q * t.estep]);
-                if (Y::G > 1 && t.z0 > 0 && t.g == 1) hx[q].x = a.in[5][zb + q * t.estep];
-            }
-        load(5, s3);
-            inv(s3);    // zeta
-            inv(hx);
-            if constexpr (Y::G == 1) {
-#pragma unroll
-                for (int q = 0; q < E; ++q) hz[q] = make_double2(t.z0 > 0 ? a.in[5][zb + q * t.estep] : 0.0, 0.0);
-                inv(hz);
-            }
-            const double vortrms = a.scal[(size_t)blockIdx.y * SC_NSCAL + SC_VORTRMS];
-            double w2 = 0.0, l1 = 0.0, l2 = 0.0;
-#pragma unroll
-            for (int q = 0; q < E; ++q) {
-                // level below 2g: the upper level of the pair below, or the halo
-                double p1 = hx[q].x, p2 = hx[q].y, p3;
-                if constexpr (Y::G > 1) {
-                    p3 = __shfl_down(hx[q].x, 1);
-                    const double u1 = __shfl_up(s1[q].y, 1), u2 = __shfl_up(s2[q].y, 1), u3 = __shfl_up(s3[q].y, 1);
-                    if (t.g > 0) {
-                        p1 = u1;
-                        p2 = u2;
-                        p3 = u3;
-                    }
-                } else {
-                    p3 = hz[q].x;
-                }
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (!(h ? t.v1 : t.v0)) continue;
-                    const double o1 = h ? s1[q].y : s1[q].x, o2 = h ? s2[q].y : s2[q].x, o3 = h ? s3[q].y : s3[q].x;
-                    w2 = fmax(w2, o1 * o1 + o2 * o2 + o3 * o3);
-                    if (h == 0 && t.z0 + 2 * t.g == 0) continue;
-                    const double t1 = fabs(0.5 * ((h ? s1[q].x : p1) + o1)), t2 = fabs(0.5 * ((h ? s2[q].x : p2) + o2)),
-                                 t3 = fabs(0.5 * ((h ? s3[q].x : p3) + o3));
-                    if (t1 + t2 + t3 > vortrms) {
-                        l1 += t1 + t2 + t3;
-                        l2 += t1 * t1 + t2 * t2 + t3 * t3;
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);   // one element at a time (registers)
-            }
-            res[RX_W2MAX] = w2;
-            res[RX_L1] = l1;
-            res[RX_L2] = l2;
-        }
-        auto into = [&](double2(&s)[E], const double2(&d)[E], double f) {   // s = d + f s
-#pragma unroll
-            for (int q = 0; q < E; ++q) s[q] = make_double2(d[q].x + f * s[q].x, d[q].y + f * s[q].y);
-        };
-            load(8, s4);
-        inv(s4);             // dw/dy
-        into(s1, s4, -0.5);  // S23
-        load(6, s5);
-        inv(s5);             // du/dy
-        into(s3, s5, 0.5);   // S12
-        load(2, s4);
-        deriv(s4);           // dw/dx
-        into(s2, s4, 0.5);   // S13
-        load(0, s5);
-        deriv(s5);           // du/dx
-        load(7, s4);
-        inv(s4);             // dv/dy
-        // p^2 of point (q, h); evaluated again where it is needed, to hold fewer registers
-#define C_(V) (h ? (V).y : (V).x)
-        auto psq = [&](int q, int h) {
-            const double x = C_(s5[q]), y = C_(s4[q]), z = x + y, b = C_(s3[q]), d = C_(s2[q]), e = C_(s1[q]);
-            return ((x * x + y * y + z * z) + 2.0 * (b * b + d * d + e * e)) * (1.0 / 6.0);
-        };
-        double pmax = 0.0;
-#pragma unroll
-        for (int q = 0; q < E; ++q)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                if (h ? t.v1 : t.v0) pmax = fmax(pmax, psq(q, h));
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) pmax = fmax(pmax, __shfl_xor(pmax, m));
-        const double cut = 0.75 * (1.0 - 1.0e-6) * pmax;
-        const bool lids = t.z0 == 0 || t.z0 + Y::LEV > nz;   // the tile has a lid (wave-uniform)
-        double gg = 2.220446049250313e-16, us = 0.0, ls = 0.0;
-#pragma unroll
-        for (int q = 0; q < E; ++q)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int z = t.z0 + 2 * t.g + h;
-                const bool lid = lids && (z == 0 || z == nz);
-                const double p2 = psq(q, h);
-                if (!((h ? t.v1 : t.v0) && (p2 >= cut || lid))) continue;
-                const double x = C_(s5[q]), y = C_(s4[q]), b = C_(s3[q]), d = C_(s2[q]), e = C_(s1[q]);
-                const double w = -(x + y);
-                const double lam = eig_absmax0(p2, x * (y * w - e * e) - b * (b * w - e * d) + d * (b * e - y * d));
-                gg = fmax(gg, lam);
-                if (z == nz) us = fmax(us, lam);
-                if (z == 0) ls = fmax(ls, lam);
-                __builtin_amdgcn_sched_barrier(0);   // one point at a time (registers)
-            }
-#undef C_
-        res[RX_GG] = gg;
-        res[RX_USGG] = us;
-        res[RX_LSGG] = ls;
-    }
-    // the block's partial; velocity maxima are the wave's already
-    __shared__ double red[kLwWaves][RX_N];
-#pragma unroll
-    for (int k = 0; k < RX_N; ++k) {
-        const bool add = k == RX_L1 || k == RX_L2;
-        if (k != RX_UMAX && k != RX_VMAX && k != RX_WMAX)
-#pragma unroll
-            for (int m = 32; m >= 1; m >>= 1) {
-                const double o = __shfl_xor(res[k], m);
-                res[k] = add ? res[k] + o : fmax(res[k], o);
-            }
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = res[k];
-    }
-    __syncthreads();
-    if (threadIdx.x < RX_N) {
-        const int k = threadIdx.x;
-        double v = red[0][k];
-#pragma unroll
-        for (int w = 1; w < kLwWaves; ++w) v = (k == RX_L1 || k == RX_L2) ? v + red[w][k] : fmax(v, red[w][k]);
-        a.part[(size_t)blockIdx.y * a.bt.part + (size_t)t.tile * RX_N + k] = v;
-    }
-}
-
-// layouts: transform-only passes, and passes that hold several fields
-using L64 = Lay<64, 8, 8, 8, 1>;
-using L128 = Lay<128, 16, 8, 16, 1>;
-using L256 = Lay<256, 16, 16, 16, 1>;
-using L512 = Lay<512, 16, 8, 8, 8>;
-using M64 = Lay<64, 8, 8, 8, 1>;
-using M128 = Lay<128, 8, 8, 4, 4>;
-using M256 = Lay<256, 8, 8, 8, 4>;
-using M512 = Lay<512, 16, 8, 8, 8>;   // (8 elements per lane, one level pair per wave: 1.5-1.7x slower)
-
-template <class Y>
-LineArgs lw_args(const LineArgs &a) {
-    LineArgs b = a;
-    b.ZC = Y::LEV * kLwWaves;
-    b.nzt = (a.g.nz + 1 + b.ZC - 1) / b.ZC;
-    return b;
-}
-template <class Y, bool FWD>
-hipError_t go_lines(const LineArgs &a, hipStream_t stream) {
-    const LineArgs b = lw_args<Y>(a);
-    hipLaunchKernelGGL((k_lw_lines<Y, FWD>), dim3(b.nother * b.nzt, b.bt.nb > 1 ? b.bt.nb : 1, b.nf),
-                       dim3(64 * kLwWaves), lw_lds<Y>(), stream, b);
-    return hipGetLastError();
-}
-template <class Y>
-hipError_t go_held(const LineArgs &a, hipStream_t stream) {
-    const LineArgs b = lw_args<Y>(a);
-    const dim3 grid(b.nother * b.nzt, b.bt.nb > 1 ? b.bt.nb : 1), block(64 * kLwWaves);
-    if (a.mode == LM_XMAIN)
-        hipLaunchKernelGGL((k_lw_xmain<Y>), grid, block, lw_lds<Y>(), stream, b);
-    else
-        hipLaunchKernelGGL((k_lw_xadapt<Y>), grid, block, lw_lds<Y>(), stream, b);
-    return hipGetLastError();
-}
-template <class Y>
-hipError_t go_inv_d(const LineArgs &a, hipStream_t stream) {
-    const LineArgs b = lw_args<Y>(a);
-    hipLaunchKernelGGL((k_lw_inv_d<Y>), dim3(b.nother * b.nzt, b.bt.nb > 1 ? b.bt.nb : 1, 6), dim3(64 * kLwWaves),
-                       lw_lds<Y>(), stream, b);
-    return hipGetLastError();
-}
-template <class Y, class M>
-hipError_t go(const LineArgs &a, hipStream_t stream) {
-    switch (a.mode) {
-        case LM_FWD: return go_lines<Y, true>(a, stream);
-        case LM_INV: return go_lines<Y, false>(a, stream);
-        case LM_INV_Y1: return go_inv_d<Y>(a, stream);
-        case LM_XMAIN:
-        case LM_XADAPT: return go_held<M>(a, stream);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-}  // namespace
-
-#define PS3D_LW_SIZES(X) X(64) X(128) X(256) X(512)
 
 // Whether a mode has a wave kernel for the line length.  (The x products pass of 512 points
 // holds six fields of 16 elements per lane, one wave per SIMD: 13.9 ms per 512^3 step
 // against 13.2 of the tile pass, which it keeps.)
 bool linewave_ok(int n, int mode) {
     if (mode == LM_DIFF || (mode == LM_XMAIN && n == 512)) return false;
-    switch (n) {
-#define CASE(N_) case N_: return true;
-        PS3D_LW_SIZES(CASE)
-#undef CASE
-        default: return false;
-    }
+    LwSet s;
+    return find_set(n, s);
 }
 int linewave_blocks(int n, int nz) {
-    int zc = 0;
-    switch (n) {
-#define CASE(N_) case N_: zc = M##N_::LEV * kLwWaves; break;
-        PS3D_LW_SIZES(CASE)
-#undef CASE
-        default: return 0;
-    }
+    LwSet s;
+    if (!find_set(n, s)) return 0;
+    const int zc = s.levels(n);
     return (nz + 1 + zc - 1) / zc;
 }
-
-hipError_t configure_linewave() {
-    hipError_t e = hipSuccess;
-#define SET(K, Y) if (e == hipSuccess) e = hipFuncSetAttribute((const void *)(K), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lw_lds<Y>());
-#define CASE(N_)                                                                                           \
-    SET((k_lw_lines<L##N_, true>), L##N_) SET((k_lw_lines<L##N_, false>), L##N_) SET((k_lw_inv_d<L##N_>), L##N_) \
-    if (linewave_ok(N_, LM_XMAIN)) SET((k_lw_xmain<M##N_>), M##N_) SET((k_lw_xadapt<M##N_>), M##N_)
-    PS3D_LW_SIZES(CASE)
-#undef CASE
-#undef SET
-    return e;
-}
-
 hipError_t launch_linewave(const LineArgs &a, hipStream_t stream) {
-    switch (a.n) {
-#define CASE(N_) case N_: return go<L##N_, M##N_>(a, stream);
-        PS3D_LW_SIZES(CASE)
-#undef CASE
-        default: return hipErrorInvalidValue;
-    }
+    LwSet s;
+    return find_set(a.n, s) ? s.launch(a, stream) : hipErrorInvalidValue;
 }
 
 }  // namespace ps3d

@@ -420,7 +420,6 @@ static int init_handle(ps3d_handle *h, const ps3d_params *p, bool alloc_fields, 
     HIPCHK(ps3d::configure_zpass());
     HIPCHK(ps3d::configure_zwave());
     HIPCHK(ps3d::configure_linepass());
-    HIPCHK(ps3d::configure_linewave());
     {   // device address of the allocation-free partials array (once per device)
         double *scr = nullptr;
         HIPCHK(ps3d::stats_scratch(h->device, &scr));
