@@ -99,6 +99,14 @@ PS3D_CPLAN8(768, 8, 8, 4, 3)
 PS3D_CPLAN8(1024, 8, 8, 4, 4)
 PS3D_CPLAN8(1536, 8, 8, 8, 3)
 PS3D_CPLAN8(2048, 8, 8, 8, 4)
+PS3D_CPLAN8(60, 5, 4, 3, 0)
+PS3D_CPLAN8(80, 8, 5, 2, 0)
+PS3D_CPLAN8(120, 8, 5, 3, 0)
+PS3D_CPLAN8(160, 8, 5, 4, 0)
+PS3D_CPLAN8(200, 8, 5, 5, 0)
+PS3D_CPLAN8(240, 8, 5, 3, 2)
+PS3D_CPLAN8(320, 8, 8, 5, 0)
+PS3D_CPLAN8(400, 8, 5, 5, 2)
 #undef PS3D_CPLAN8
 
 // LDS slot of line element x.  SKEW: one pad slot after every 16 elements, so that

@@ -41,7 +41,7 @@ static int fail(int code, const std::string &msg) {
     } while (0)
 
 namespace ps3d {
-hipError_t configure_zpass();
+hipError_t configure_zpass(const ZLaunch &zl);
 hipError_t configure_linepass();
 }
 
@@ -417,7 +417,7 @@ static int init_handle(ps3d_handle *h, const ps3d_params *p, bool alloc_fields, 
         h->lsy = line_sched_ok(ny, sy) ? sy : line_sched_default(ny);
     }
 
-    HIPCHK(ps3d::configure_zpass());
+    HIPCHK(ps3d::configure_zpass(h->zl));
     HIPCHK(ps3d::configure_zwave());
     HIPCHK(ps3d::configure_linepass());
     {   // device address of the allocation-free partials array (once per device)

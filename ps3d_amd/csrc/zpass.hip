@@ -1370,7 +1370,12 @@ static inline int zbatch(const ZOpArgs &) { return 1; }
 static inline int zbatch(const ZStageArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1; }
 
 // (ZPT, nz) pairs with a compile-time FFT plan; other nz use the runtime plan.
-#define PS3D_Z_SIZES(X) X(1, 32) X(1, 48) X(1, 64) X(1, 96) X(1, 128) X(1, 192) X(1, 256) X(1, 384) \
+// Depths with a compile-time plan: 2^a 3^b and those with one or two factors of 5 that a
+// column of one level per thread takes.  Against the run-time plan (per-pass switch on the
+// radix, divisions by the pass's span) tendency + next vor2vel take 0.143 for 0.183 ms per
+// 100^3 step, 0.667 for 0.791 at 160^3, 1.139 for 1.408 at 200^3, 48 for 63 us at 30^3.
+#define PS3D_Z_SIZES(X) X(1, 30) X(1, 32) X(1, 40) X(1, 48) X(1, 60) X(1, 80) X(1, 100) X(1, 120) X(1, 160) X(1, 200) \
+    X(1, 64) X(1, 96) X(1, 128) X(1, 192) X(1, 256) X(1, 384) \
     X(2, 512) X(2, 768) X(3, 1024)
 
 #define ZLAUNCH(KERNEL, Z_, N_, ARGS, LAUNCH) \
@@ -1414,13 +1419,17 @@ hipError_t launch_zstage(const ZLaunch &zl, int kind, const ZStageArgs &args, hi
     return done ? hipGetLastError() : hipErrorInvalidValue;
 }
 
-hipError_t configure_zpass() {
+hipError_t configure_zpass(const ZLaunch &zl) {   // the kernels that one depth can take
     const int lds = 160 * 1024;
     hipError_t e = hipSuccess;
 #define SETA(K) \
     if (e == hipSuccess) e = hipFuncSetAttribute((const void *)(K), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
 #define ZST_SET(Z_, N_, M_) SETA((k_zstage<Z_, N_, M_>))
-#define ZCFG3(Z_, N_) SETA((k_zinv<Z_, N_>)) SETA((k_ztend<Z_, N_>)) SETA((k_zop<Z_, N_>)) ZST_KINDS(ZST_SET, Z_, N_)
+#define ZCFG3(Z_, N_)                                                      \
+    if (zl.zpt == Z_ && (N_ == 0 || zl.nz == N_)) {                        \
+        SETA((k_zinv<Z_, N_>)) SETA((k_ztend<Z_, N_>)) SETA((k_zop<Z_, N_>)) \
+        ZST_KINDS(ZST_SET, Z_, N_)                                         \
+    }
     PS3D_Z_SIZES(ZCFG3)
     ZCFG3(1, 0) ZCFG3(2, 0) ZCFG3(3, 0)
     SETA(k_zrk<1>) SETA(k_zrk<2>) SETA(k_zrk<3>)

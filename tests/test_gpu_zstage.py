@@ -61,3 +61,24 @@ def test_semi_spectral_steps_match_the_passes_on_svor(monkeypatch, shape, filter
     close(a.get(G.SVOR), b.get(G.SVOR))
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("nz", [30, 40, 60, 80, 100, 120, 160, 200])
+def test_depths_with_a_factor_of_5_match_the_oracle(oracle_mod, nz):
+    """Both steppers, three steps on the compile-time plans of these depths, to the
+    trajectories' parity tolerance."""
+    from ps3d_amd import gpu as G
+    print("z plan", nz, flush=True)
+    shape = (8, 6, nz)
+    for stepper in ("impl-diff-rk4", "cn2"):
+        kw = dict(BOX, stepper=stepper, filtering="Hou & Li", nnu=3, prediss=30.0, pretype="vorch",
+                  length_scale="Kolmogorov")
+        o = oracle_mod.Oracle(oracle_mod.make_params(*shape, **kw))
+        d = G.Ps3dGpu(G.make_params(*shape, **kw))
+        w = ics.beltrami_multimode(*shape, seed=4)
+        for s in (o, d):
+            s.set_vorticity(w)
+        o.advance_n(3), d.advance_n(3)
+        close(d.get(G.SVOR), o.get(oracle_mod.SVOR))
+        o.close()
+        d.close()
