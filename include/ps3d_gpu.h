@@ -180,7 +180,8 @@ int ps3d_gpu_advance_until(ps3d_handle *h, double *t, double t_stop, int nmax, d
  * the last ps3d_gpu_vor2vel; call it after vor2vel (and adapt) and before source,
  * where write_step sits in advance (advance.f90:85-91).  Neither field feeds the
  * time step, so ps3d_gpu_advance_n leaves them out; results are read with
- * PS3D_PRES / PS3D_DELTA. */
+ * PS3D_PRES / PS3D_DELTA.  Not between the stages of a step made of
+ * ps3d_gpu_rk_substep calls, whose initial state it overwrites. */
 int ps3d_gpu_derived(ps3d_handle *h);
 
 /* = update_netcdf_field_diagnostics (src/fields/field_diagnostics_netcdf.f90:257-439)

@@ -81,6 +81,7 @@ struct ps3d_handle {
     // passes of the operator entry points, vor2vel and tendency on svor, for comparison
     bool zfuse = true;
     bool svor_semi = false;        // svor holds combined columns (between such steps)
+    bool substep_open = false;     // qdi, qdf hold a step that ps3d_gpu_rk_substep has begun
     int kxb = 0, kyb = 0;          // largest wavenumber indices the tendency filter passes
     LineCfg lx{}, ly{};
     // tiles of the register-holding line modes (x products pass lxm, x adapt pass lxr,
@@ -698,10 +699,27 @@ static int ensure_semi(ps3d_handle *h) {
     return 0;
 }
 
+// Before steps: svor in their form; a substep sequence the caller has left ends.
+static int begin_steps(ps3d_handle *h) {
+    h->substep_open = false;
+    return ensure_semi(h);
+}
+
+// svor into the mixed form, in place.
+static int ensure_mixed(ps3d_handle *h) {
+    for (int c = 0; c < 3 && h->svor_semi; ++c)
+        HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->svor[c]), h->stream));
+    h->svor_semi = false;
+    return 0;
+}
+
 // The mixed form of svor, for the host and for other grids: svor itself, or decomposed
-// into qdi (which carries data only inside the steps on svor).  The state stays as it is.
+// into qdi, the state staying as it is.  Between two substeps of ps3d_gpu_rk_substep qdi
+// carries the step's initial state; svor is then decomposed in place, as the next substep
+// would do.
 static int mixed_svor(ps3d_handle *h, double *const **src) {
     *src = h->svor;
+    if (h->substep_open) return ensure_mixed(h);
     if (!h->svor_semi) return 0;
     for (int c = 0; c < 3; ++c)
         HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->qdi[c]), h->stream));
@@ -1027,6 +1045,7 @@ static ps3d_handle make_view(const ps3d_handle *h, int b) {
     v.zl = h->zl;
     v.zfuse = h->zfuse;
     v.svor_semi = h->svor_semi;
+    v.substep_open = h->substep_open;
     v.kxb = h->kxb;
     v.kyb = h->kyb;
     v.TQ = h->TQ; v.QPB = h->QPB; v.nquads = h->nquads;
@@ -1104,6 +1123,7 @@ int ps3d_gpu_set_vorticity(ps3d_handle *h, const double *vor) {
     if ((st = line_fields(h, 1, LM_FWD, 3, h->vel, h->vel))) return st;
     if ((st = line_fields(h, 0, LM_FWD, 3, h->vel, h->svor))) return st;
     h->svor_semi = semi_steps(h);
+    h->substep_open = false;
     if (!h->svor_semi)
         for (int c = 0; c < 3; ++c)
             HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->svor[c]), h->stream));
@@ -1215,7 +1235,7 @@ int ps3d_gpu_step(ps3d_handle *h, double *t, double dt) {
     HIPCHK(hipMemcpyAsync(h->scal + SC_DT, &dt, sizeof(double), hipMemcpyHostToDevice, h->stream));
     const int mode = h->p.stepper == PS3D_STEPPER_CN2 ? ZT_CN2 : ZT_RK4;
     const bool semi = mode == ZT_RK4 && semi_steps(h);
-    if ((st = ensure_semi(h))) return st;
+    if ((st = begin_steps(h))) return st;
     if (semi) {
         HIPCHK(launch_zstage(h->zl, ZS_STEP, zstage_args(h, 1, h->mid), h->stream));
     } else {
@@ -1296,7 +1316,7 @@ int ps3d_gpu_advance_n(ps3d_handle *h, double *t, int nsteps, double *diag_serie
     if (!h || !t || nsteps < 0) return fail(PS3D_E_ARG, "invalid argument");
     if (!h->have_state) return fail(PS3D_E_STATE, "advance before set_vorticity");
     int st;
-    if ((st = ensure_semi(h))) return st;
+    if ((st = begin_steps(h))) return st;
     if ((st = ensure_diag(h, std::max(1, nsteps)))) return st;
     double zero = 0.0;
     HIPCHK(hipMemcpyAsync(h->scal + SC_T, t, sizeof(double), hipMemcpyHostToDevice, h->stream));
@@ -1323,7 +1343,7 @@ int ps3d_gpu_advance_until(ps3d_handle *h, double *t, double t_stop, int nmax, d
     if (!h->have_state) return fail(PS3D_E_STATE, "advance before set_vorticity");
     if (h->cnn) return fail(PS3D_E_UNSUPPORTED, "advance_until with a closure attached: use ps3d_gpu_advance_n");
     int st;
-    if ((st = ensure_semi(h))) return st;
+    if ((st = begin_steps(h))) return st;
     if ((st = ensure_diag(h, std::max(1, nmax)))) return st;
     // SC_STEP, SC_GATE, SC_TSTOP are consecutive slots
     const double init[3] = {0.0, 0.0, std::min(t_stop, h->p.limit)};
@@ -1347,13 +1367,12 @@ int ps3d_gpu_rk_substep(ps3d_handle *h, int stage, double dt, const double *vdis
     HIPCHK(hipMemcpyAsync(h->scal + SC_DT, &dt, sizeof(double), hipMemcpyHostToDevice, h->stream));
     ZTendArgs a = ztend_args(h, ZT_RK4, stage, nullptr);
     a.rk.vdiss = dv;
-    hipError_t e = hipSuccess;
-    for (int c = 0; c < 3 && h->svor_semi && e == hipSuccess; ++c)   // the substep takes the mixed form
-        e = launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->svor[c]), h->stream);
-    h->svor_semi = false;
-    if (e == hipSuccess) e = launch_zrk(h->zl, a, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    const int st = ensure_mixed(h);   // the substep takes the mixed form
+    hipError_t e = st ? hipSuccess : launch_zrk(h->zl, a, h->stream);
+    if (!st && e == hipSuccess) e = hipStreamSynchronize(h->stream);
     (void)hipFree(dv);
+    if (st) return st;
+    h->substep_open = stage < 4;
     if (e != hipSuccess) return fail(PS3D_E_HIP, std::string("rk_substep: ") + hipGetErrorString(e));
     return 0;
 }
@@ -1363,7 +1382,7 @@ int ps3d_gpu_profile_kernels(ps3d_handle *h, int nsteps, double *ms, int *launch
     if (!h || nsteps < 1) return fail(PS3D_E_ARG, "invalid argument");
     if (!h->have_state) return fail(PS3D_E_STATE, "profile before set_vorticity");
     int st;
-    if ((st = ensure_semi(h))) return st;
+    if ((st = begin_steps(h))) return st;
     if ((st = ensure_diag(h, nsteps))) return st;
     double zero = 0.0;
     HIPCHK(hipMemcpyAsync(h->scal + SC_STEP, &zero, sizeof(double), hipMemcpyHostToDevice, h->stream));
@@ -1428,7 +1447,8 @@ int ps3d_gpu_last_timing(ps3d_handle *h, double *ms, int *nsteps) {
 
 // pressure + horizontal_divergence (fields_derived.f90:67-182) from the state of the
 // last vor2vel: svel (semi-spectral), vor and the y-derivatives du/dy, dv/dy, dw/dy
-// (physical).  qdi / qdf serve as scratch: they only carry data inside a step.
+// (physical).  qdi / qdf serve as scratch: they only carry data inside a step (one made of
+// ps3d_gpu_rk_substep calls has to be complete).
 int ps3d_gpu_derived(ps3d_handle *h) {
     if (h && h->nbatch != 1) return fail(PS3D_E_STATE, "batched handle: use the _batch entry points");
     if (!h) return fail(PS3D_E_ARG, "null handle");
@@ -1895,6 +1915,7 @@ int ps3d_gpu_resample(ps3d_handle *dst, ps3d_handle *src, int which) {
     }
     dst->have_state = true;
     dst->svor_semi = false;
+    dst->substep_open = false;
     return finish_setup(dst);
 }
 
@@ -1929,6 +1950,7 @@ int ps3d_gpu_set_vorticity_batch(ps3d_handle *h, int b, const double *vor) {
     int st = ps3d_gpu_set_vorticity(&v, vor);
     if (st) return st;
     h->inst_set[b] = 1;
+    h->substep_open = false;
     h->svor_semi = semi_steps(h);   // an instance without a state is zero in either form
     h->have_state = std::all_of(h->inst_set.begin(), h->inst_set.end(), [](char c) { return c != 0; });
     h->have_phys = h->have_adapt = h->have_grad = false;
@@ -1939,7 +1961,9 @@ int ps3d_gpu_get_batch(ps3d_handle *h, int b, int which, double *host) {
     if (!h || !host || b < 0 || b >= h->nbatch) return fail(PS3D_E_ARG, "invalid argument");
     if (which != PS3D_SVOR) return fail(PS3D_E_UNSUPPORTED, "batched handles hold svor between steps");
     ps3d_handle v = make_view(h, b);
-    return ps3d_gpu_get(&v, which, host);
+    const int st = ps3d_gpu_get(&v, which, host);
+    if (h->nbatch == 1) h->svor_semi = v.svor_semi;   // decomposed in place during a substep sequence
+    return st;
 }
 
 // Enqueues nsteps fused steps of every instance (no host synchronisation).
