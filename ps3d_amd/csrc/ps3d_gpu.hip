@@ -1999,6 +1999,7 @@ int ps3d_gpu_advance_n_batch(ps3d_handle *h, double *t, int nsteps, double *diag
     if (!h || !t || nsteps < 0) return fail(PS3D_E_ARG, "invalid argument");
     if (!h->have_state) return fail(PS3D_E_STATE, "advance before every instance has an initial vorticity");
     int st;
+    if ((st = begin_steps(h))) return st;
     if (diag_series && (st = ensure_diag(h, std::max(1, nsteps)))) return st;
     if ((st = put_times(h, t))) return st;
     HIPCHK(hipEventRecord(h->ev0, h->stream));
@@ -2121,6 +2122,11 @@ int ps3d_gpu_ensemble_advance(ps3d_ensemble *e, int nsteps, int use_graph, doubl
     for (ps3d_handle *h : e->g)
         if (!h->have_state) return fail(PS3D_E_STATE, "advance before every instance has an initial vorticity");
     int st;
+    for (ps3d_handle *h : e->g) {
+        const bool wait = semi_steps(h) && !h->svor_semi;
+        if ((st = begin_steps(h))) return st;
+        if (wait) HIPCHK(hipStreamSynchronize(h->stream));   // a replay on s0 is not ordered behind this stream
+    }
     if (use_graph && e->exec) {
         // a group's captured arguments changed (its diagnostics buffer was
         // reallocated by advance_n_batch, say): capture again
@@ -2185,6 +2191,7 @@ int ps3d_gpu_ensemble_tune(ps3d_ensemble *e, int steps, int *choice) {
     for (size_t gi = 0; gi < e->g.size(); ++gi) {
         ps3d_handle *h = e->g[gi];
         if (!h->have_state) return fail(PS3D_E_STATE, "tune needs the initial vorticity of every instance");
+        if ((st = begin_steps(h))) return st;
         const size_t nb = h->nbatch, sv = 3 * h->nvol;
         double *bk = nullptr;
         HIPCHK(hipMalloc((void **)&bk, sizeof(double) * (sv * nb + SC_NSCAL * nb + h->b_roll * nb)));
