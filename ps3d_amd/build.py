@@ -4,9 +4,12 @@ Fortran host program ps3d_driver on top of it with amdflang.
 Usage: python -m ps3d_amd.build [--verbose]
 """
 import concurrent.futures as cf
+import glob
 import os
 import subprocess
 import sys
+
+from .lanecheck import misplaced_spills
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -32,13 +35,25 @@ CFLAGS = [
 
 
 def _compile(src, verbose=False, extra=()):
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC] + CFLAGS + list(extra) + ["-c", os.path.join(CSRC, src), "-o", obj]
+    stem = os.path.splitext(src)[0]
+    obj = os.path.join(BUILD, stem + ".o")
+    cmd = [HIPCC] + CFLAGS + list(extra) + (["-save-temps=obj"] if src.endswith(".hip") else []) + ["-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("hipcc failed for %s:\n%s\n%s" % (src, " ".join(cmd), r.stderr[-8000:]))
     if verbose and r.stderr.strip():
         sys.stderr.write(r.stderr)
+    temps = glob.glob(os.path.join(BUILD, stem + "-h*")) + glob.glob(os.path.join(BUILD, stem + ".hip-*"))
+    bad = []
+    for listing in temps:
+        if listing.endswith(ARCH + ".s"):
+            with open(listing) as f:
+                bad += misplaced_spills(f.read())
+    for t in temps:
+        os.remove(t)
+    if bad:
+        os.remove(obj)
+        raise RuntimeError("%s: spills with lanes switched off (lanecheck.py): %s" % (src, bad))
     return obj
 
 
