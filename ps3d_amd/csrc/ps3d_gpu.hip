@@ -919,53 +919,77 @@ static int one_step(ps3d_handle *h) {
 // Host <-> device copies between ps3d's (0:nz, y, x) layout and the padded columns.
 // A strided 2-D copy from pageable memory moves one short row at a time; instead whole
 // padded columns go through pinned staging buffers in large contiguous copies, and the
-// (un)padding is a memcpy per column on the host.  Volumes of many chunks are shared by
+// (un)padding is a memcpy per column on the host.  What fits the first buffer takes one
+// wait for all its volumes.  More is cut into chunks of kChunkBytes, shared by
 // kCopyThreads threads with a buffer each: one core's memcpy and page faults held the copy
 // to 10 GB/s, with eight the others' copies overlap it (a state to the host: 512^3 285 ->
 // 71 ms, 45 GB/s; 256^3 40 -> 10 ms; 128^3 5.5 -> 2.1 ms).  The buffers are the process's,
 // under one lock.
 namespace {
-constexpr size_t kStageBytes = 4u << 20;
+constexpr size_t kStageBytes = 16u << 20, kChunkBytes = 4u << 20;
 constexpr int kCopyThreads = 8;
 std::mutex g_stage_mu;
-double *g_stage[kCopyThreads] = {};
+double *g_stage[kCopyThreads] = {};   // of kStageBytes, then kChunkBytes
+
+// one column at a time, in functions of their own: as loops over captured references they
+// took 2 ns more a column, 3-16 % of the small copies
+void pad_columns(double *stage, const double *u, size_t nc, size_t nz1, size_t zs) {
+    for (size_t c = 0; c < nc; ++c, stage += zs, u += nz1) {
+        std::memcpy(stage, u, sizeof(double) * nz1);
+        std::memset(stage + nz1, 0, sizeof(double) * (zs - nz1));
+    }
+}
+void unpad_columns(double *u, const double *stage, size_t nc, size_t nz1, size_t zs) {
+    for (size_t c = 0; c < nc; ++c, stage += zs, u += nz1) std::memcpy(u, stage, sizeof(double) * nz1);
+}
 }  // namespace
+
+static int stage_buffer(int i, size_t bytes) {
+    if (!g_stage[i] && hipHostMalloc((void **)&g_stage[i], bytes, hipHostMallocDefault) != hipSuccess) {
+        g_stage[i] = nullptr;
+        return fail(PS3D_E_NOMEM, "pinned staging buffer");
+    }
+    return 0;
+}
 
 // nf volumes dev[0..nf-1] <-> host, back to back there.
 static int copy_fields(ps3d_handle *h, int nf, double *const *dev, double *host, bool to_host) {
     std::lock_guard<std::mutex> lk(g_stage_mu);
     const size_t nz1 = (size_t)h->g.nz + 1, zs = h->g.zs, ncol = (size_t)h->g.nx * h->g.ny;
-    const size_t cpc = std::min(ncol, std::max<size_t>(1, kStageBytes / (sizeof(double) * zs)));
+    int st;
+    if ((st = stage_buffer(0, kStageBytes))) return st;   // (a column is 8 KB at most)
+    if (nf * ncol * zs * sizeof(double) <= kStageBytes) {
+        // (a field's volumes follow each other on the device too)
+        const size_t bytes = sizeof(double) * nf * ncol * zs;
+        if (!to_host) pad_columns(g_stage[0], host, nf * ncol, nz1, zs);
+        HIPCHK(to_host ? hipMemcpyAsync(g_stage[0], dev[0], bytes, hipMemcpyDeviceToHost, h->stream)
+                       : hipMemcpyAsync(dev[0], g_stage[0], bytes, hipMemcpyHostToDevice, h->stream));
+        HIPCHK(hipStreamSynchronize(h->stream));
+        if (to_host) unpad_columns(host, g_stage[0], nf * ncol, nz1, zs);
+        return 0;
+    }
+    const size_t cpc = std::min(ncol, kChunkBytes / (sizeof(double) * zs));
     const size_t per = (ncol + cpc - 1) / cpc, njob = per * nf;
-    // a thread costs some 20 us to start: from about 8 MB each has two chunks or more
+    // a thread costs some 20 us to start: each has two chunks or more
     const int nt = (int)std::min<size_t>(kCopyThreads, std::max<size_t>(1, njob / 2));
-    for (int i = 0; i < nt; ++i)
-        if (!g_stage[i] && hipHostMalloc((void **)&g_stage[i], std::max(kStageBytes, sizeof(double) * zs), hipHostMallocDefault) != hipSuccess) {
-            g_stage[i] = nullptr;
-            if (i == 0) return fail(PS3D_E_NOMEM, "pinned staging buffer");
-        }
+    for (int i = 1; i < nt; ++i)
+        if (!g_stage[i] && hipHostMalloc((void **)&g_stage[i], kChunkBytes, hipHostMallocDefault) != hipSuccess) g_stage[i] = nullptr;
     std::atomic<size_t> next{0};
     std::atomic<int> err{0};
     auto work = [&](double *stage, bool own_thread) {
         hipEvent_t ev = nullptr;
         hipError_t e = own_thread ? hipSetDevice(h->device) : hipSuccess;
-        if (e == hipSuccess && nt > 1) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
         for (size_t j; e == hipSuccess && err.load() == 0 && (j = next.fetch_add(1)) < njob;) {
             const size_t c0 = j % per * cpc, nc = std::min(cpc, ncol - c0), bytes = sizeof(double) * nc * zs;
             double *d = dev[j / per] + c0 * zs, *u = host + (j / per * ncol + c0) * nz1;
-            if (!to_host)
-                for (size_t c = 0; c < nc; ++c) {
-                    std::memcpy(stage + c * zs, u + c * nz1, sizeof(double) * nz1);
-                    std::memset(stage + c * zs + nz1, 0, sizeof(double) * (zs - nz1));
-                }
+            if (!to_host) pad_columns(stage, u, nc, nz1, zs);
             e = to_host ? hipMemcpyAsync(stage, d, bytes, hipMemcpyDeviceToHost, h->stream)
                         : hipMemcpyAsync(d, stage, bytes, hipMemcpyHostToDevice, h->stream);
-            // the buffer is read or refilled next: wait for this copy (alone on the stream,
-            // for the stream: 15 us less than an event's creation and wait)
-            if (e == hipSuccess && ev) e = hipEventRecord(ev, h->stream);
-            if (e == hipSuccess) e = ev ? hipEventSynchronize(ev) : hipStreamSynchronize(h->stream);
-            if (e == hipSuccess && to_host)
-                for (size_t c = 0; c < nc; ++c) std::memcpy(u + c * nz1, stage + c * zs, sizeof(double) * nz1);
+            // the buffer is read or refilled next: wait for this copy
+            if (e == hipSuccess) e = hipEventRecord(ev, h->stream);
+            if (e == hipSuccess) e = hipEventSynchronize(ev);
+            if (e == hipSuccess && to_host) unpad_columns(u, stage, nc, nz1, zs);
         }
         if (ev) (void)hipEventDestroy(ev);
         if (e != hipSuccess) err.store((int)e);
@@ -1736,9 +1760,7 @@ int ps3d_gpu_get(ps3d_handle *h, int which, double *host) {
     }
     const int nc = (which == PS3D_PRES || which == PS3D_DELTA) ? 1 : 3;
     int st;
-    if ((st = copy_fields(h, nc, src, host, true))) return st;
-    HIPCHK(hipStreamSynchronize(h->stream));
-    return 0;
+    return copy_fields(h, nc, src, host, true);
 }
 
 int ps3d_gpu_set(ps3d_handle *h, int which, const double *host) {
@@ -1751,9 +1773,7 @@ int ps3d_gpu_set(ps3d_handle *h, int which, const double *host) {
         default: return fail(PS3D_E_UNSUPPORTED, "field cannot be set");
     }
     int st;
-    if ((st = copy_fields(h, 3, dst, const_cast<double *>(host), false))) return st;
-    HIPCHK(hipStreamSynchronize(h->stream));
-    return 0;
+    return copy_fields(h, 3, dst, const_cast<double *>(host), false);
 }
 
 int ps3d_gpu_op(ps3d_handle *h, int op, const double *in, double *out) {
@@ -1795,9 +1815,7 @@ int ps3d_gpu_op(ps3d_handle *h, int op, const double *in, double *out) {
         default:
             return fail(PS3D_E_ARG, "unknown op");
     }
-    if ((st = copy_out(h, out, res))) return st;
-    HIPCHK(hipStreamSynchronize(h->stream));
-    return 0;
+    return copy_out(h, out, res);
 }
 
 // Batched stafft transforms on x(m, n) (m fastest) through the line / z kernels.
