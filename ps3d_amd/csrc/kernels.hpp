@@ -145,6 +145,8 @@ struct ZOpArgs {
     const double *in;
     double *out;
     int op;
+    int nvol;                 // volumes, vol doubles apart in both in and out
+    long vol;
 };
 
 struct MeanArgs {

@@ -664,7 +664,18 @@ static ZOpArgs zop_args(ps3d_handle *h, int op, const double *in, double *out) {
     a.in = in;
     a.out = out;
     a.op = op;
+    a.nvol = 1;
     return a;
+}
+
+// One z operator on the three volumes of a field, in one launch (as three, the combine or
+// decompose of a small grid's state took 30 us instead of 10): a field's volumes follow each
+// other in the pool.
+static hipError_t launch_zop3(ps3d_handle *h, int op, double *const *in, double *const *out) {
+    ZOpArgs a = zop_args(h, op, in[0], out[0]);
+    a.nvol = 3;
+    a.vol = (long)h->nvol;
+    return launch_zop(h->zl, a, h->stream);
 }
 
 static int run_mean(ps3d_handle *h, int mode, int advance_time, double *const *svor = nullptr) {
@@ -693,8 +704,7 @@ static bool semi_steps(const ps3d_handle *h) { return h->zfuse && h->p.stepper =
 // mixed form there (set_vorticity, resample, set): the columns combined.
 static int ensure_semi(ps3d_handle *h) {
     if (!semi_steps(h) || h->svor_semi) return 0;
-    for (int c = 0; c < 3; ++c)
-        HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_COMBINE, h->svor[c], h->svor[c]), h->stream));
+    HIPCHK(launch_zop3(h, ZOP_COMBINE, h->svor, h->svor));
     h->svor_semi = true;
     return 0;
 }
@@ -707,8 +717,7 @@ static int begin_steps(ps3d_handle *h) {
 
 // svor into the mixed form, in place.
 static int ensure_mixed(ps3d_handle *h) {
-    for (int c = 0; c < 3 && h->svor_semi; ++c)
-        HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->svor[c]), h->stream));
+    if (h->svor_semi) HIPCHK(launch_zop3(h, ZOP_DECOMPOSE, h->svor, h->svor));
     h->svor_semi = false;
     return 0;
 }
@@ -721,8 +730,7 @@ static int mixed_svor(ps3d_handle *h, double *const **src) {
     *src = h->svor;
     if (h->substep_open) return ensure_mixed(h);
     if (!h->svor_semi) return 0;
-    for (int c = 0; c < 3; ++c)
-        HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->qdi[c]), h->stream));
+    HIPCHK(launch_zop3(h, ZOP_DECOMPOSE, h->svor, h->qdi));
     *src = h->qdi;
     return 0;
 }
@@ -879,9 +887,7 @@ static int fused_stage(ps3d_handle *h, int mode, int stage) {
         if ((st = line_fields(h, 1, LM_FWD, 3, h->grad, h->grad))) return st;
         if ((st = line_fields(h, 0, LM_FWD, 3, h->grad, h->grad))) return st;
         // the passes on svor add it decomposed (mid is free after the adapt stage)
-        if (!semi)
-            for (int c = 0; c < 3; ++c)
-                HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->grad[c], h->mid[c]), h->stream));
+        if (!semi) HIPCHK(launch_zop3(h, ZOP_DECOMPOSE, h->grad, h->mid));
     }
     if (semi) {
         ZStageArgs z = zstage_args(h, stage, rqp);
@@ -1148,9 +1154,7 @@ int ps3d_gpu_set_vorticity(ps3d_handle *h, const double *vor) {
     if ((st = line_fields(h, 0, LM_FWD, 3, h->vel, h->svor))) return st;
     h->svor_semi = semi_steps(h);
     h->substep_open = false;
-    if (!h->svor_semi)
-        for (int c = 0; c < 3; ++c)
-            HIPCHK(launch_zop(h->zl, zop_args(h, ZOP_DECOMPOSE, h->svor[c], h->svor[c]), h->stream));
+    if (!h->svor_semi) HIPCHK(launch_zop3(h, ZOP_DECOMPOSE, h->svor, h->svor));
     return finish_setup(h);
 }
 

@@ -1160,7 +1160,7 @@ __global__ void __launch_bounds__(512) k_zrk(ZTendArgs a) {
 template <int ZPT, int NZ>
 __global__ void __launch_bounds__(512) k_zop(ZOpArgs a) {
     const Grid g = a.g;
-    ZT<ZPT> T = make_zt<ZPT>(g, a.tb, a.TQ, a.QPB, a.nquads);
+    ZT<ZPT> T = make_zt<ZPT>(g, a.tb, a.TQ, a.QPB, a.nquads, (long)blockIdx.y * a.vol);
     ZLds L = zlds(a.QPB, T.N, g.nz);
     double F[ZPT][4], O[ZPT][4];
     zload(T, a.in, F);
@@ -1366,7 +1366,7 @@ size_t zpass_lds_bytes(int QPB, int nz) {
 
 static inline int zbatch(const ZInvArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1; }
 static inline int zbatch(const ZTendArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1; }
-static inline int zbatch(const ZOpArgs &) { return 1; }
+static inline int zbatch(const ZOpArgs &a) { return a.nvol; }
 static inline int zbatch(const ZStageArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1; }
 
 // (ZPT, nz) pairs with a compile-time FFT plan; other nz use the runtime plan.

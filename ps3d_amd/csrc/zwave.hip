@@ -1372,7 +1372,7 @@ __global__ void __launch_bounds__(256) k_zop_w(ZOpArgs a) {
     constexpr int S = WDim<NZ>::S, P = WDim<NZ>::P;
     extern __shared__ double2 wsm[];
     const Grid g = a.g;
-    const WC c = make_wc(g, a.tb, 0);
+    const WC c = make_wc(g, a.tb, (long)blockIdx.y * a.vol);
     double2 *ws = wsm + (size_t)c.m * WDim<NZ>::WS;
     const WTw<P> tw = make_tw<P>(a.twz, c.lane);
     const double sc = a.zscale;
@@ -1517,7 +1517,7 @@ hipError_t launch_zstage_w(int nz, int nquads, int kind, const ZStageArgs &a, hi
     return hipGetLastError();
 }
 hipError_t launch_zop_w(int nz, int nquads, const ZOpArgs &args, hipStream_t stream) {
-    ZW_DISPATCH(k_zop_w, nquads, 1, args);
+    ZW_DISPATCH(k_zop_w, nquads, args.nvol, args);
     return hipGetLastError();
 }
 
