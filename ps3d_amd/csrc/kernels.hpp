@@ -268,6 +268,8 @@ int line_reg_zc(int n, int T);
 hipError_t launch_line(const LineArgs &a, int nthreads, hipStream_t stream);
 // Line passes with the lines in a wave's registers (linewave.hip)
 bool linewave_ok(int n, int mode);
+// the x products pass: points of a field over all instances, physical or spectral input
+bool linewave_xmain(int n, size_t points, bool phys_in);
 int linewave_blocks(int n, int nz);   // blocks per line set of LM_XMAIN / LM_XADAPT (a partial each)
 hipError_t launch_linewave(const LineArgs &a, hipStream_t stream);
 

@@ -1079,7 +1079,9 @@ bool line_sched_ok(int n, int sched) {
 
 hipError_t launch_line(const LineArgs &a, int nthreads, hipStream_t stream) {
     (void)nthreads;
-    if (a.lw && linewave_ok(a.n, a.mode)) return launch_linewave(a, stream);
+    const size_t points = (size_t)a.g.nx * a.g.ny * (a.g.nz + 1) * (a.bt.nb > 1 ? a.bt.nb : 1);
+    if (a.lw && (a.mode == LM_XMAIN ? linewave_xmain(a.n, points, a.phys_in) : linewave_ok(a.n, a.mode)))
+        return launch_linewave(a, stream);
     // compile-time plans need the standard tile depth of their build
     const bool reg = a.mode == LM_INV_Y1 || a.mode == LM_XMAIN || a.mode == LM_XADAPT;
     const int rt = (a.rthreads == 512 || a.rthreads == 256) ? a.rthreads : kLineThreads;

@@ -809,7 +809,9 @@ static int x_adapt(ps3d_handle *h, int phys_in, bool velmax_given = false) {
     if (x.lw) f.nbx = h->lxr.nother * linewave_blocks(h->g.nx, h->g.nz);
     if (velmax_given) {
         f.partm = h->partm;
-        f.nbm = h->lxm.nother * (h->lw && linewave_ok(h->g.nx, LM_XMAIN) ? linewave_blocks(h->g.nx, h->g.nz) : h->lxm.nzt);
+        const size_t points = (size_t)h->g.nx * h->g.ny * (h->g.nz + 1) * h->nbatch;
+        f.nbm = h->lxm.nother *
+                (h->lw && linewave_xmain(h->g.nx, points, false) ? linewave_blocks(h->g.nx, h->g.nz) : h->lxm.nzt);
     }
     prof_begin(h, PS3D_K_REDUCE);
     HIPCHK(launch_fin_x(f, h->stream));
