@@ -14,9 +14,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -955,6 +955,7 @@ void unpad_columns(double *u, const double *stage, size_t nc, size_t nz1, size_t
 static int stage_buffer(int i, size_t bytes) {
     if (!g_stage[i] && hipHostMalloc((void **)&g_stage[i], bytes, hipHostMallocDefault) != hipSuccess) {
         g_stage[i] = nullptr;
+        (void)hipGetLastError();   // not an error of the launches that follow
         return fail(PS3D_E_NOMEM, "pinned staging buffer");
     }
     return 0;
@@ -978,10 +979,10 @@ static int copy_fields(ps3d_handle *h, int nf, double *const *dev, double *host,
     }
     const size_t cpc = std::min(ncol, kChunkBytes / (sizeof(double) * zs));
     const size_t per = (ncol + cpc - 1) / cpc, njob = per * nf;
-    // a thread costs some 20 us to start: each has two chunks or more
-    const int nt = (int)std::min<size_t>(kCopyThreads, std::max<size_t>(1, njob / 2));
+    // a thread costs some 20 us to start: each has two chunks or more, and a buffer
+    int nt = (int)std::min<size_t>(kCopyThreads, std::max<size_t>(1, njob / 2));
     for (int i = 1; i < nt; ++i)
-        if (!g_stage[i] && hipHostMalloc((void **)&g_stage[i], kChunkBytes, hipHostMallocDefault) != hipSuccess) g_stage[i] = nullptr;
+        if (stage_buffer(i, kChunkBytes)) nt = i;
     std::atomic<size_t> next{0};
     std::atomic<int> err{0};
     auto work = [&](double *stage, bool own_thread) {
@@ -1005,8 +1006,8 @@ static int copy_fields(ps3d_handle *h, int nf, double *const *dev, double *host,
     std::thread pool[kCopyThreads];
     int started = 0;
     try {
-        for (int i = 1; i < nt && g_stage[i]; ++i, ++started) pool[i] = std::thread(work, g_stage[i], true);
-    } catch (const std::system_error &) {   // no more threads: the others take the chunks
+        for (int i = 1; i < nt; ++i, ++started) pool[i] = std::thread(work, g_stage[i], true);
+    } catch (const std::exception &) {   // no more threads or memory: the others take the chunks
     }
     work(g_stage[0], false);
     for (int i = 1; i <= started; ++i) pool[i].join();
