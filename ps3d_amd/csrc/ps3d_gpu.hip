@@ -952,6 +952,17 @@ void unpad_columns(double *u, const double *stage, size_t nc, size_t nz1, size_t
 }
 }  // namespace
 
+// Makes a device the thread's current one for a while.
+struct OnDevice {
+    int before = 0;
+    hipError_t e;
+    explicit OnDevice(int device) {
+        e = hipGetDevice(&before);
+        if (e == hipSuccess && before != device) e = hipSetDevice(device);
+    }
+    ~OnDevice() { (void)hipSetDevice(before); }
+};
+
 static int stage_buffer(int i, size_t bytes) {
     if (!g_stage[i] && hipHostMalloc((void **)&g_stage[i], bytes, hipHostMallocDefault) != hipSuccess) {
         g_stage[i] = nullptr;
@@ -985,9 +996,10 @@ static int copy_fields(ps3d_handle *h, int nf, double *const *dev, double *host,
         if (stage_buffer(i, kChunkBytes)) nt = i;
     std::atomic<size_t> next{0};
     std::atomic<int> err{0};
-    auto work = [&](double *stage, bool own_thread) {
+    auto work = [&](double *stage) {
+        const OnDevice on(h->device);   // the event is recorded on this device's stream
         hipEvent_t ev = nullptr;
-        hipError_t e = own_thread ? hipSetDevice(h->device) : hipSuccess;
+        hipError_t e = on.e;
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
         for (size_t j; e == hipSuccess && err.load() == 0 && (j = next.fetch_add(1)) < njob;) {
             const size_t c0 = j % per * cpc, nc = std::min(cpc, ncol - c0), bytes = sizeof(double) * nc * zs;
@@ -1006,10 +1018,10 @@ static int copy_fields(ps3d_handle *h, int nf, double *const *dev, double *host,
     std::thread pool[kCopyThreads];
     int started = 0;
     try {
-        for (int i = 1; i < nt; ++i, ++started) pool[i] = std::thread(work, g_stage[i], true);
+        for (int i = 1; i < nt; ++i, ++started) pool[i] = std::thread(work, g_stage[i]);
     } catch (const std::exception &) {   // no more threads or memory: the others take the chunks
     }
-    work(g_stage[0], false);
+    work(g_stage[0]);
     for (int i = 1; i <= started; ++i) pool[i].join();
     if (err.load()) return fail(PS3D_E_HIP, std::string("field copy: ") + hipGetErrorString((hipError_t)err.load()));
     return 0;

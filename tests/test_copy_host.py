@@ -71,3 +71,15 @@ except G.Ps3dError as e:
 d = handle(*SMALL)
 assert stub.hipGetLastError() == 0
 """, STUB_HOST_ALLOCS="0")
+
+
+def test_a_handle_of_another_device_than_the_current_one(run):
+    """The handle's stream and the copies' events belong to its device, whichever device the
+    calling thread has current; that stays current."""
+    run("""
+d = handle(*LARGE)
+assert stub.hipSetDevice(1) == 0
+same(d)
+now = C.c_int()
+assert stub.hipGetDevice(C.byref(now)) == 0 and now.value == 1
+""")
