@@ -23,7 +23,6 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 
 PEAK_HBM = 8.0e12          # MI355X HBM3E, B/s
-B_STEP_VOLUMES = 218       # algorithmic full-volume FP64 touches per RK4 step (fused floor)
 KIND_NAMES = ["zinv", "yinv", "xmain", "yfwd", "ztend", "yinv_adapt", "xadapt", "reduce", "mean", "ztend_zinv"]
 
 
@@ -73,6 +72,25 @@ def workload_params(mod, n):
                            filtering="2/3-rule", stepper="impl-diff-rk4", nnu=3, prediss=30.0,
                            pretype="vorch", length_scale="Kolmogorov", alpha=0.1, dt_fixed=0.0,
                            limit=1.0e30)
+
+
+def profile_step(G, h, steps):
+    """(ms, launches, algorithmic bytes per launch) of every kernel kind over `steps` steps."""
+    import ctypes as C
+    import numpy as np
+    ms = np.zeros(len(KIND_NAMES))
+    launches = np.zeros(len(KIND_NAMES), dtype=np.int32)
+    nbytes = np.zeros(len(KIND_NAMES))
+    if G.lib().ps3d_gpu_profile_kernels(h.h, steps, ms.ctypes.data_as(C.c_void_p), launches.ctypes.data_as(C.c_void_p),
+                                        nbytes.ctypes.data_as(C.c_void_p)):
+        raise RuntimeError(G.lib().ps3d_gpu_last_error().decode())
+    return ms, launches, nbytes
+
+
+def step_bytes(G, h):
+    """Bytes the kernels of one step have to move: what each launch reads and writes, once."""
+    _, launches, nbytes = profile_step(G, h, 1)
+    return float((launches * nbytes).sum())
 
 
 def read_traffic(n):
@@ -134,9 +152,12 @@ def ensemble_bench(G, steps, sep_steps):
     for h in sep:
         h.advance_n(sep_steps)
     el_sep = time.perf_counter() - t0
+    b_step, i = 0.0, 0
+    for c in ENSEMBLE_COUNTS:
+        b_step += c * step_bytes(G, sep[i])
+        i += c
     for h in sep:
         h.close()
-    b_step = B_STEP_VOLUMES * 8.0 * npts
     return {
         "instances": ntot, "sizes": ENSEMBLE_SIZES, "counts": ENSEMBLE_COUNTS, "npts_total": npts,
         "ic": "random-phase isotropic, k0 ~ U[2,6] per instance (numpy PCG64 seed 2024), IC seeds 1000+i",
@@ -210,10 +231,10 @@ def configs_bench(G, ics):
         t0 = time.perf_counter()
         d.advance_n(steps)
         el = time.perf_counter() - t0
+        b_step = step_bytes(G, d)
         d.close()
         npts = n * n * (n + 1)
         sps = steps / el
-        b_step = B_STEP_VOLUMES * 8.0 * npts
         out.append({"config": label, "grid": [n, n, n], "steps": steps, "steps_per_s": sps,
                     "ms_per_step": 1e3 * el / steps, "grid_point_updates_per_s": npts * sps,
                     "step_roofline_frac": b_step * sps / PEAK_HBM})
@@ -331,21 +352,14 @@ def main():
     npts = n * n * (n + 1)
 
     # per-kernel durations (HIP events on the handle's stream), outside the timed region
-    import ctypes as C
-    import numpy as np
-    ms = np.zeros(len(KIND_NAMES))
-    launches = np.zeros(len(KIND_NAMES), dtype=np.int32)
-    nbytes = np.zeros(len(KIND_NAMES))
-    st = G.lib().ps3d_gpu_profile_kernels(d.h, a.profile_steps, ms.ctypes.data_as(C.c_void_p),
-                                          launches.ctypes.data_as(C.c_void_p), nbytes.ctypes.data_as(C.c_void_p))
+    ms, launches, nbytes = profile_step(G, d, a.profile_steps)
     kernels = {}
-    if st == 0:
-        for k, name in enumerate(KIND_NAMES):
-            if launches[k]:
-                avg = ms[k] / launches[k] * 1e-3
-                kernels[name] = {"ms_per_step": ms[k] / a.profile_steps, "avg_launch_us": avg * 1e6,
-                                 "algo_bytes": nbytes[k],
-                                 "gbs": (nbytes[k] / avg / 1e9) if nbytes[k] > 0 else None}
+    for k, name in enumerate(KIND_NAMES):
+        if launches[k]:
+            avg = ms[k] / launches[k] * 1e-3
+            kernels[name] = {"ms_per_step": ms[k] / a.profile_steps, "avg_launch_us": avg * 1e6,
+                             "algo_bytes": nbytes[k],
+                             "gbs": (nbytes[k] / avg / 1e9) if nbytes[k] > 0 else None}
     dom = max((k for k in kernels if kernels[k]["algo_bytes"] > 0), key=lambda k: kernels[k]["ms_per_step"],
               default=None)
     traffic = read_traffic(n)
@@ -355,7 +369,7 @@ def main():
         roofline = {"bound": "hbm", "kernel": dom, "achieved": achieved / 1e9, "peak": PEAK_HBM / 1e9,
                     "unit": "GB/s", "frac": achieved / PEAK_HBM,
                     "traffic": traffic.get(dom)}
-    b_step = B_STEP_VOLUMES * 8.0 * npts
+    b_step = float((launches * nbytes).sum()) / a.profile_steps
     out = {
         "metric": "RK steps/s at %d^3 FP64" % n,
         "value": steps_per_s,

@@ -1457,7 +1457,7 @@ int ps3d_gpu_profile_kernels(ps3d_handle *h, int nsteps, double *ms, int *launch
         bytes[PS3D_K_ZINV] = (cn2 ? (14.0 + 2 * 9.0) / 3.0 : (14.0 + 3 * 9.0) / 4.0) * vol;
         bytes[PS3D_K_YINV] = 12.0 * vol;        // 6 R + 6 W
         // shares of the kx slots and of the columns that the tendency filter passes
-        const bool semi = semi_steps(h);
+        const bool semi = semi_steps(h), wave = wave_adapt(h);
         const double bx = semi ? std::min(1.0, (2.0 * h->kxb + 1.0) / h->g.nx) : 1.0;
         const double band = semi ? bx * std::min(1.0, (2.0 * h->kyb + 1.0) / h->g.ny) : 1.0;
         bytes[PS3D_K_XMAIN] = (6.0 + 3.0 * bx) * vol;           // 6 R + 3 W
@@ -1469,12 +1469,13 @@ int ps3d_gpu_profile_kernels(ps3d_handle *h, int nsteps, double *ms, int *launch
             // stage 1: 3 R a0, 6 W + band (3 R, 3 W); stages 2, 3 also read qdf
             bytes[PS3D_K_ZTEND_ZINV] = (9.0 + band * (6.0 + 2 * 9.0) / 3.0) * vol;
             bytes[PS3D_K_ZTEND] = (6.0 + band * 3.0) * vol;
-            bytes[PS3D_K_ZINV] = 12.0 * vol;
+            bytes[PS3D_K_ZINV] = (wave ? 9.0 : 12.0) * vol;     // 3 R + 6 W (and 3 W midpoints)
         }
-        bytes[PS3D_K_YINV_ADAPT] = 21.0 * vol;  // 9 R + 12 W
-        // x adapt in a step: 11 R (u, w for their x derivatives, the y derivatives,
-        // omega, the midpoints); the velocity maxima come from the products pass
-        bytes[PS3D_K_XADAPT] = 11.0 * vol;
+        bytes[PS3D_K_YINV_ADAPT] = (wave ? 15.0 : 21.0) * vol;  // 6 R + 9 W; with the midpoints 9 R + 12 W
+        // x adapt in a step: 8 R (u, w for their x derivatives, the y derivatives, omega)
+        // and the midpoints where the pass does not form them; the velocity maxima come
+        // from the products pass
+        bytes[PS3D_K_XADAPT] = (wave ? 8.0 : 11.0) * vol;
         bytes[PS3D_K_REDUCE] = 0.0;
         bytes[PS3D_K_MEAN] = 0.0;
     }
