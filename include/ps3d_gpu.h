@@ -323,23 +323,25 @@ int ps3d_gpu_ensemble_group(ps3d_ensemble *e, int g, ps3d_handle **h);
 /* nsteps steps of every instance of every group; use_graph = 1 replays one
  * captured graph per step.  ms: kernel time (HIP events), may be NULL. */
 int ps3d_gpu_ensemble_advance(ps3d_ensemble *e, int nsteps, int use_graph, double *ms);
-/* Times `steps` steps of each group under each available z launch shape and
- * keeps the fastest, then, one mode at a time, the block size of each
- * register-holding line pass, then the FFT schedule of the transform-only y and x
- * line passes (state restored afterwards).  choice[g] (may be
+/* Times `steps` steps of each group under each z launch shape that changes its step
+ * (the register variants differ for cn2 only) and keeps the fastest, then, for the
+ * line passes that run on tiles (lengths without a wave kernel, cn2's adapt stage,
+ * small grids' x products), one mode at a time, the block size of each
+ * register-holding pass and the FFT schedule of the transform-only y and x passes
+ * (state restored afterwards).  choice[g] (may be
  * NULL) receives the shape code: 100..102 = one wavefront per column (register
  * budget variant), q < 100 = q quads per block of the quad-per-thread kernels. */
 int ps3d_gpu_ensemble_tune(ps3d_ensemble *e, int steps, int *choice);
 int ps3d_gpu_ensemble_set_choice(ps3d_ensemble *e, int g, int code);
 /* Block sizes (threads) the tuner chose for group g's register-holding line passes:
  * threads[0] x products, [1] adapt-stage y, [2] x adapt (1024, 512 or 256: full,
- * half or quarter tile depth).  No counterpart in the reference. */
+ * half or quarter tile depth); the fixed rule's where a pass is not on tiles.  No counterpart in the reference. */
 int ps3d_gpu_ensemble_line_choice(ps3d_ensemble *e, int g, int *threads);
 /* FFT schedules the tuner chose for group g's transform-only line passes:
  * sched[0] x lines, sched[1] y lines; bit 1 = radix-8-first plan (else
  * radix-16-first), bit 2 = the Hermitian pair of the inverse formed in the first
- * radix pass (else a pass of its own), bit 4 = 512 threads per tile (else 256).
- * No counterpart in the reference. */
+ * radix pass (else a pass of its own), bit 4 = 512 threads per tile (else 256);
+ * the fixed rule's where these passes are not on tiles.  No counterpart in the reference. */
 int ps3d_gpu_ensemble_fft_schedule(ps3d_ensemble *e, int g, int *sched);
 int ps3d_gpu_ensemble_destroy(ps3d_ensemble *e);
 

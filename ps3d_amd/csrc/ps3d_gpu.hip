@@ -741,6 +741,11 @@ static bool wave_adapt(const ps3d_handle *h) {
     return h->lw && semi_steps(h) && linewave_ok(h->g.nx, LM_XADAPT) && linewave_ok(h->g.ny, LM_INV_Y1);
 }
 
+// Whether a step's x products pass takes its wave kernel (launch_line).
+static bool wave_products(const ps3d_handle *h) {
+    return h->lw && linewave_xmain(h->g.nx, (size_t)h->g.nx * h->g.ny * (h->g.nz + 1) * h->nbatch, false);
+}
+
 // vor2vel + the adapt-stage y pass: leaves u, v, w, xi, eta, zeta, their y
 // derivatives and z midpoints x-spectral / y-physical, svel semi-spectral, svor
 // projected and the Parseval sums finished into scal.
@@ -809,9 +814,7 @@ static int x_adapt(ps3d_handle *h, int phys_in, bool velmax_given = false) {
     if (x.lw) f.nbx = h->lxr.nother * linewave_blocks(h->g.nx, h->g.nz);
     if (velmax_given) {
         f.partm = h->partm;
-        const size_t points = (size_t)h->g.nx * h->g.ny * (h->g.nz + 1) * h->nbatch;
-        f.nbm = h->lxm.nother *
-                (h->lw && linewave_xmain(h->g.nx, points, false) ? linewave_blocks(h->g.nx, h->g.nz) : h->lxm.nzt);
+        f.nbm = h->lxm.nother * (wave_products(h) ? linewave_blocks(h->g.nx, h->g.nz) : h->lxm.nzt);
     }
     prof_begin(h, PS3D_K_REDUCE);
     HIPCHK(launch_fin_x(f, h->stream));
@@ -2221,6 +2224,26 @@ static void apply_z_choice(ps3d_handle *h, int code) {
 
 static int current_z_choice(const ps3d_handle *h) { return h->zl.wave ? 99 + h->zl.wave : h->QPB; }
 
+// The candidates that differ in a step: RK4's stage kernels have one wave build, which every
+// wave code selects (cn2's passes have one per code).
+static std::vector<int> step_z_candidates(const ps3d_handle *h) {
+    std::vector<int> c = z_candidates(h);
+    if (semi_steps(h) && ps3d::zwave_supported(h->g.nz)) {
+        const int wave = h->zl.wave ? current_z_choice(h) : 101;
+        c.erase(std::remove_if(c.begin(), c.end(), [wave](int v) { return v >= 100 && v != wave; }), c.end());
+    }
+    return c;
+}
+
+// Which line passes of a step run on tiles, whose block sizes and schedules are tuned: 0 the x
+// products pass, 1 the adapt stage along y, 2 along x; the transform-only passes along an axis.
+static bool tile_pass(const ps3d_handle *h, int mode) {
+    return mode == 0 ? !wave_products(h) : !wave_adapt(h);
+}
+static bool tile_transforms(const ps3d_handle *h, int axis) {
+    return !(h->lw && linewave_ok(axis == 0 ? h->g.nx : h->g.ny, LM_FWD));
+}
+
 // Times `steps` fused steps of each group under every candidate shape and keeps the
 // fastest; the state (svor, device scalars, rolling-mean history) is restored.
 int ps3d_gpu_ensemble_tune(ps3d_ensemble *e, int steps, int *choice) {
@@ -2239,7 +2262,7 @@ int ps3d_gpu_ensemble_tune(ps3d_ensemble *e, int steps, int *choice) {
                                   h->stream));
         HIPCHK(hipMemcpyAsync(bsc, h->scal, sizeof(double) * SC_NSCAL * nb, hipMemcpyDeviceToDevice, h->stream));
         HIPCHK(hipMemcpyAsync(brl, h->roll, sizeof(double) * h->b_roll * nb, hipMemcpyDeviceToDevice, h->stream));
-        const std::vector<int> cand = z_candidates(h);
+        const std::vector<int> cand = step_z_candidates(h);
         int best = current_z_choice(h);
         float best_ms = 1e30f;
         for (int code : cand) {
@@ -2261,6 +2284,7 @@ int ps3d_gpu_ensemble_tune(ps3d_ensemble *e, int steps, int *choice) {
         if (!st) {
             int cur[3] = {h->rtm, h->rty, h->rtx};
             for (int mode = 0; mode < 3 && !st; ++mode) {
+                if (!tile_pass(h, mode)) continue;
                 int bestT = cur[mode];
                 float bt = 1e30f;
                 for (int T : {1024, 512, 256}) {
@@ -2286,6 +2310,7 @@ int ps3d_gpu_ensemble_tune(ps3d_ensemble *e, int steps, int *choice) {
         }
         // FFT schedule of the transform-only passes: y lines, then x lines
         for (int axis = 1; axis >= 0 && !st; --axis) {
+            if (!tile_transforms(h, axis)) continue;
             const int n = axis == 0 ? h->g.nx : h->g.ny;
             int &cur = axis == 0 ? h->lsx : h->lsy;
             int bests = cur;

@@ -392,8 +392,8 @@ class Ps3dEnsemble:
         return ms.value
 
     def tune(self, steps=2):
-        """z launch shape, then line-pass block sizes, per group; returns the z shape
-        codes (line_choices() gives the block sizes)."""
+        """z launch shape, then block sizes and schedules of the line passes on tiles, per
+        group; returns the z shape codes (line_choices() gives the block sizes)."""
         ch = (C.c_int * len(self.groups))()
         _check(lib().ps3d_gpu_ensemble_tune(self.e, int(steps), ch))
         return list(ch)

@@ -12,7 +12,7 @@
 namespace {
 thread_local int cur = 0;
 thread_local hipError_t last = hipSuccess;
-std::atomic<int> host_calls{0};
+std::atomic<int> host_calls{0}, launches{0};
 struct Obj { int dev; };
 hipError_t ret(hipError_t e) {
     if (e != hipSuccess) last = e;
@@ -32,6 +32,7 @@ hipError_t alloc(void **p, size_t n) {
 
 extern "C" {
 int stub_host_calls() { return host_calls; }
+int stub_launches() { return launches; }
 
 hipError_t hipGetDevice(int *d) { return *d = cur, hipSuccess; }
 hipError_t hipSetDevice(int d) { return d < 0 || d > 1 ? ret(hipErrorInvalidDevice) : (cur = d, hipSuccess); }
@@ -71,7 +72,7 @@ hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 0.0f, hipSuccess; }
 
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return ++launches, hipSuccess; }
 hipError_t hipGetSymbolAddress(void **p, const void *) {
     static double scratch[8];
     return *p = scratch, hipSuccess;
