@@ -124,7 +124,12 @@ struct ZStageArgs {
     int kxb, kyb;
     const double *in[3];      // ZS_STEP: svorts (mixed); ZS_STAGE*: r, q, p (semi-spectral)
     double *svor[3];          // the state at the step's start; ZS_STAGE4 writes the new one
-    double *qdf[3];           // the accumulated result
+    // the step's accumulated tendency, without the state, which it joins in the last stage.
+    // Added to the state stage by stage, each addition rounded the combined columns at their
+    // full size: error against 64-bit arithmetic after 20 steps (128^3: 30) 1.5, 1.8, 2.2, 3.0
+    // and 6.0e-15 at 32^3, 48^3, 64^3, 96^3 and 128^3, so 1.15, 1.4, 1.6, 2.0 and 3.9e-15; the
+    // mixed state, whose interior coefficients are small, 1.3, 1.6, 1.9, 2.3 and 4.8e-15.
+    double *qdf[3];
     double *out[6];           // u, v, w, xi, eta, zeta; ZS_START: out[3..5] = svor (projected)
     // ZS_START, for the adapt stage: the z-midpoint vorticity of the tile passes, or the
     // Parseval sums (RY_*) of each block; nullptr: left out

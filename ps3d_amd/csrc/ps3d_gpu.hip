@@ -1471,7 +1471,8 @@ int ps3d_gpu_profile_kernels(ps3d_handle *h, int nsteps, double *ms, int *launch
             // only the columns in the band read r, q, p and carry qdf
             // stage 1: 3 R a0, 6 W + band (3 R, 3 W); stages 2, 3 also read qdf
             bytes[PS3D_K_ZTEND_ZINV] = (9.0 + band * (6.0 + 2 * 9.0) / 3.0) * vol;
-            bytes[PS3D_K_ZTEND] = (6.0 + band * 3.0) * vol;
+            // last stage: 3 R a0, 3 W + band (6 R)
+            bytes[PS3D_K_ZTEND] = (6.0 + band * 6.0) * vol;
             bytes[PS3D_K_ZINV] = (wave ? 9.0 : 12.0) * vol;     // 3 R + 6 W (and 3 W midpoints)
         }
         bytes[PS3D_K_YINV_ADAPT] = (wave ? 15.0 : 21.0) * vol;  // 6 R + 9 W; with the midpoints 9 R + 12 W

@@ -859,9 +859,12 @@ __device__ __attribute__((always_inline)) inline void zsolve(const ZStageArgs &a
     }
 }
 
-// (one level per thread fits four waves per SIMD without spills)
+// Waves per SIMD at one level per thread: three without spills for the first and the last
+// stage (the last at four spills 140 bytes a lane: 31 us for 20 at 96^3), four for stages 1 to
+// 3, which spill 52 to 112 bytes a lane there.
 template <int ZPT, int NZ, int M>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ZPT > 1 || M == ZS_STEP ? 1 : M == ZS_START ? 3 : 4, 8)))
+__global__ void __launch_bounds__(512)
+__attribute__((amdgpu_waves_per_eu(ZPT > 1 || M == ZS_STEP ? 1 : M == ZS_START || M == ZS_STAGE4 ? 3 : 4, 8)))
 k_zstage(ZStageArgs a) {
     const Grid &g = a.g;
     if (gated_off(g.gate)) return;
@@ -876,7 +879,7 @@ k_zstage(ZStageArgs a) {
         zsolve<ZPT, NZ>(a, T, L, F[0], F[1], F[2]);
     } else {
         // coefficients of the substep (impl_rk4.f90:37-53, 87-89, 212-364):
-        // q = mul (a0 + ca f t), qdf += cb f t
+        // q = mul (a0 + ca f t), qdf += cb f t; last: q = mul (a0 + (qdf + ca f t))
         const double dt = scal[SC_DT];
         const double f0 = T.q00 ? 1.0 : (a.tb.hou_li ? exp(a.tb.filx[T.kx] + a.tb.fily[T.ky])
                                                      : a.tb.filx[T.kx] * a.tb.fily[T.ky]);
@@ -910,7 +913,7 @@ k_zstage(ZStageArgs a) {
 #pragma unroll
                     for (int m = 0; m < 4; ++m) {
                         const double a0 = F[k][s][m], sq = f * S[k][s][m];
-                        S[k][s][m] = a0 + cb * sq;
+                        S[k][s][m] = cb * sq;
                         F[k][s][m] = mul * (a0 + ca * sq);
                     }
                 zstore(T, a.qdf[k], S[k]);
@@ -937,8 +940,8 @@ k_zstage(ZStageArgs a) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 double X[ZPT][4], B[ZPT][4];
-                zload(T, M == ZS_STAGE4 && band ? a.qdf[k] : a.svor[k], F[k]);
-                if (M == ZS_STAGE23 && band) zload(T, a.qdf[k], B);
+                zload(T, a.svor[k], F[k]);
+                if (M != ZS_STAGE1 && band) zload(T, a.qdf[k], B);
                 if (band && a.extra[0]) zload(T, a.extra[k], X);
 #pragma unroll
                 for (int s = 0; s < ZPT; ++s)
@@ -950,8 +953,9 @@ k_zstage(ZStageArgs a) {
                                           : T.fx[m] * Q[s][m ^ 1] - T.fy[m] * Pp[s][m ^ 2];
                         if (band && a.extra[0]) t += X[s][m];
                         const double sq = band ? f * t : nf, a0 = F[k][s][m];
-                        B[s][m] = (M == ZS_STAGE23 && band ? B[s][m] : a0) + cb * sq;
-                        F[k][s][m] = mul * (a0 + ca * sq);
+                        const double sum = M != ZS_STAGE1 && band ? B[s][m] : 0.0;
+                        if (M != ZS_STAGE4) B[s][m] = sum + cb * sq;
+                        F[k][s][m] = mul * (a0 + (M == ZS_STAGE4 ? sum + ca * sq : ca * sq));
                     }
                 if (M != ZS_STAGE4 && band) zstore(T, a.qdf[k], B);
             }

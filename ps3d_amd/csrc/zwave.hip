@@ -1272,7 +1272,7 @@ k_zstage_w(ZStageArgs a) {
                 for (int s = 0; s <= S; ++s) {
                     double &q = s < S ? F[k].v[s % S] : F[k].top;
                     const double sq = r.f0 * (s < S ? T[k].v[s % S] : T[k].top);
-                    (s < S ? Q.v[s % S] : Q.top) = q + dt6 * sq;
+                    (s < S ? Q.v[s % S] : Q.top) = dt6 * sq;
                     q = (q + dt2 * sq) * r.em;
                 }
                 wstore(c, a.qdf[k], Q);
@@ -1286,7 +1286,7 @@ k_zstage_w(ZStageArgs a) {
         const bool band = c.kx <= a.kxb && c.ky <= a.kyb;   // block-uniform
         const WRk r = wrk_setup_from<NZ>(c, rk, ZT_RK4, a.tb, wrk_inputs(c, rk, a.tb));
         const double em2 = r.em * r.em;
-        // q = mul (a0 + ca f t), qdf += cb f t (impl_rk4.f90:212-364)
+        // q = mul (a0 + ca f t), qdf += cb f t; last: q = mul (a0 + (qdf + ca f t)) (impl_rk4.f90:212-364)
         const double ca = M == ZS_STAGE4 ? r.dt / 6.0 : (M == ZS_STAGE1 || a.stage == 2 ? 0.5 * r.dt : r.dt);
         const double mul = M == ZS_STAGE4 ? em2 : (M == ZS_STAGE1 || a.stage == 2 ? r.em : em2);
         if (band) {
@@ -1305,7 +1305,7 @@ k_zstage_w(ZStageArgs a) {
             wdiff(c, g, P, FP);
             WF<NZ> A[3];
 #pragma unroll
-            for (int k = 0; k < 3; ++k) wload(c, M == ZS_STAGE4 ? a.qdf[k] : a.svor[k], A[k]);
+            for (int k = 0; k < 3; ++k) wload(c, a.svor[k], A[k]);
             __syncthreads();
             const double *r2 = sslot<NZ>(wsm, c.m ^ 2, 0, false), *r1 = sslot<NZ>(wsm, c.m ^ 1, 0, false);
             const double *q1 = sslot<NZ>(wsm, c.m ^ 1, 1, false), *p2 = sslot<NZ>(wsm, c.m ^ 2, 2, false);
@@ -1313,7 +1313,7 @@ k_zstage_w(ZStageArgs a) {
             for (int k = 0; k < 3; ++k) {
                 WF<NZ> X, D;
                 if (a.extra[0]) wload(c, a.extra[k], X);
-                if (M == ZS_STAGE23) wload(c, a.qdf[k], D);
+                if (M != ZS_STAGE1) wload(c, a.qdf[k], D);
 #pragma unroll
                 for (int s = 0; s <= S; ++s) {
                     const int z = s < S ? c.lane + 64 * s : NZ;
@@ -1323,17 +1323,21 @@ k_zstage_w(ZStageArgs a) {
                     if (a.extra[0]) t += s < S ? X.v[s % S] : X.top;
                     const double sq = f * t;
                     const double a0 = s < S ? A[k].v[s % S] : A[k].top;
-                    const double b0 = M == ZS_STAGE23 ? (s < S ? D.v[s % S] : D.top) : a0;
-                    if (M != ZS_STAGE4) (s < S ? D.v[s % S] : D.top) = b0 + cb * sq;
-                    (s < S ? F[k].v[s % S] : F[k].top) = mul * (a0 + ca * sq);
+                    double &sum = s < S ? D.v[s % S] : D.top;
+                    if (M == ZS_STAGE4) {
+                        (s < S ? F[k].v[s % S] : F[k].top) = mul * (a0 + (sum + ca * sq));
+                    } else {
+                        sum = M == ZS_STAGE1 ? cb * sq : sum + cb * sq;
+                        (s < S ? F[k].v[s % S] : F[k].top) = mul * (a0 + ca * sq);
+                    }
                 }
                 if (M != ZS_STAGE4) wstore(c, a.qdf[k], D);
             }
             // one region: the next exchange writes the slots just read
             if constexpr (!XB && M != ZS_STAGE4) __syncthreads();
         } else {
-            // no tendency here: qdf stays a0, which is all that is kept of such a column
-            // (0 * KE carries a non-finite state into it, as the filtered products would)
+            // no tendency here, and no qdf (0 * KE carries a non-finite state into the
+            // column, as the filtered products would)
             const double nf = 0.0 * a.scal[(size_t)blockIdx.y * SC_NSCAL + SC_KE];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {

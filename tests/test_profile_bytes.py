@@ -26,7 +26,7 @@ X, XY = "43 / 64", "(43 / 64) ** 2"
 # xi, eta, zeta -> u, v, w and the projected vorticity, no midpoints; y inverse of the six and
 # the derivatives of three; omega, three y derivatives, and u, w for their x derivatives
 WAVES = {"ZINV": "9", "YINV": "12", "XMAIN": "6 + 3 * " + X, "YFWD": "3 * %s + 3 * %s" % (X, XY),
-         "ZTEND": "6 + 3 * " + XY, "YADAPT": "15", "XADAPT": "8",
+         "ZTEND": "6 + 6 * " + XY, "YADAPT": "15", "XADAPT": "8",
          "ZSTAGE": "9 + %s * (6 + 9 + 9) / 3" % XY}
 # tiles: the midpoints of omega are three more fields from the z to the x pass
 TILES = dict(WAVES, ZINV="12", YADAPT="21", XADAPT="11")
