@@ -244,7 +244,10 @@ int ps3d_gpu_field_stats_noalloc(ps3d_handle *h, const double *diag, double *sta
  * be NULL. */
 int ps3d_gpu_viscosity(ps3d_handle *h, double *visc, double *pref);
 
-/* Device <-> host copies of a field (enum ps3d_field). */
+/* Device <-> host copies of a field (enum ps3d_field).  RK4 handles keep svor with its
+ * columns combined (semi-spectral) between steps: get forms PS3D_SVOR from it and leaves
+ * the state as it is, and steps combine what set has put there.  A state that is read and
+ * put back thus continues to rounding (2e-14), not bit for bit. */
 int ps3d_gpu_get(ps3d_handle *h, int which, double *host);
 int ps3d_gpu_set(ps3d_handle *h, int which, const double *host);
 

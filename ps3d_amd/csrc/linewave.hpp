@@ -28,8 +28,9 @@
 // stage along y 0.93 -> 0.58, 0.18 -> 0.062, and along x 0.75 -> 0.54, 0.155 -> 0.092.  The
 // transform-only passes run at 4.4 to 5.1 TB/s (a plain copy: 5.0).
 // The two-butterfly engine, whole RK4 steps: 96^3 0.65 -> 0.53 ms, 100^3 1.80 -> 0.63, 160^3
-// 5.40 -> 2.22, 200^3 10.2 -> 4.5, 320^3 39.7 -> 21.0, 384^3 41.6 -> 33.3; 32^3 0.223 -> 0.181,
-// where the products pass alone is slower (49 -> 66 us: few waves, one long chain each).
+// 5.40 -> 2.22, 200^3 10.2 -> 4.5, 320^3 39.7 -> 21.0, 384^3 41.6 -> 33.3; 32^3 0.223 -> 0.167,
+// with the products pass on tiles, as on small grids in general (linewave_xmain).  At 90 points
+// and above the passes that hold several fields run one wave per SIMD.
 //
 // Exchanges move real and imaginary parts one after the other through half the LDS, which
 // leaves room for four waves per SIMD.

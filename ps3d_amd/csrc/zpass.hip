@@ -1373,11 +1373,10 @@ static inline int zbatch(const ZTendArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1;
 static inline int zbatch(const ZOpArgs &a) { return a.nvol; }
 static inline int zbatch(const ZStageArgs &a) { return a.bt.nb > 1 ? a.bt.nb : 1; }
 
-// (ZPT, nz) pairs with a compile-time FFT plan; other nz use the runtime plan.
-// Depths with a compile-time plan: 2^a 3^b and those with one or two factors of 5 that a
-// column of one level per thread takes.  Against the run-time plan (per-pass switch on the
-// radix, divisions by the pass's span) tendency + next vor2vel take 0.143 for 0.183 ms per
-// 100^3 step, 0.667 for 0.791 at 160^3, 1.139 for 1.408 at 200^3, 48 for 63 us at 30^3.
+// (ZPT, nz) pairs with a compile-time FFT plan; every other depth (24, 36, 50, 54, 72, 90,
+// 108, 144, 150, 180, ... of one level per thread) uses the run-time plan.  Against that one
+// (per-pass switch on the radix, divisions by the pass's span) tendency + next vor2vel take
+// 0.143 for 0.183 ms per 100^3 step, 0.667 for 0.791 at 160^3, 1.139 for 1.408 at 200^3, 48 for 63 us at 30^3.
 #define PS3D_Z_SIZES(X) X(1, 30) X(1, 32) X(1, 40) X(1, 48) X(1, 60) X(1, 80) X(1, 100) X(1, 120) X(1, 160) X(1, 200) \
     X(1, 64) X(1, 96) X(1, 128) X(1, 192) X(1, 256) X(1, 384) \
     X(2, 512) X(2, 768) X(3, 1024)

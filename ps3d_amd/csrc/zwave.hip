@@ -983,9 +983,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NZ <=
 // factors are this member's with the sign turned.  Two exchanges are left in the
 // vor2vel part (xi, eta, d zeta/dz together; then dw/dz and zeta), one in the tendency.
 // Measured per call at 256^3 (tendency, substep and vor2vel of the passes on svor in one
-// kernel before: 800 us): stage 1 366 us, stages 2 and 3 444 us; last stage 382 -> 232 us;
-// first pass 505 -> 421 us.  512^3: 10.1 -> 4.2 and 4.8 ms.  What bounds them now is memory:
-// 4.4 TB/s at 256^3 (stages 2, 3: 14.4 volumes) with three waves per SIMD.
+// kernel before: 800 us): stages 1 to 3 400 us on average; last stage 382 -> 238 us; first
+// pass 505 -> 368 us.  512^3: 10.1 -> 4.3 ms.  What bounds them now is memory: 4.2 TB/s at
+// 256^3 in stages 1 to 3 with three waves per SIMD (the last stage: three, 4.9 TB/s; the first:
+// two, 3.3 TB/s); at 512^3 3.1 TB/s, two waves and 236 bytes a lane of spills.
 // ---------------------------------------------------------------------------
 // Region 0: the wave's FFT slice; region 1 (XB): three fields per member beside the
 // slices, where the LDS leaves room for it at full occupancy (nz <= 128): the exchange of
@@ -1223,8 +1224,10 @@ __device__ __attribute__((always_inline)) inline void wsolve(const ZStageArgs &a
     }
 }
 
-// waves per SIMD the stage kernels are built for: as many as their registers allow
-// without spills (the first pass holds the vorticity to the end for the sums)
+// Waves per SIMD the stage kernels are built for: as many as their registers allow without
+// spills (the first pass holds the vorticity to the end for the sums), but at nz = 512, where
+// stages 1 to 3 at two waves with 236 bytes a lane of spills measured faster than at one
+// (13.97 -> 12.8 ms per 512^3 step).
 constexpr int wstage_occ(int nz, int m) {
     const bool more = m == ZS_STEP || m == ZS_START;
     return nz <= 64 ? 4 : nz <= 128 ? (more ? 3 : 4) : nz <= 256 ? (more ? 2 : 3) : (more ? 1 : 2);
